@@ -313,7 +313,7 @@ __device__ __forceinline__ void poll_store(const AoLaunch &L, uint32_t gid, floa
 // another of them, so no poll sees what another one does in this round.
 __global__ void k_poll_stages(AoLaunch L) {
   for (uint32_t g = kAoRayGen; g <= kAoMiss; g++) tg::begin_phase(L.gr.g[g]);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *L.work = 0u;  // for the next round's traversal
+  if (blockIdx.x == 0) clear_work(L.work, threadIdx.x);  // for the next round's traversal
   poll_raygen(L);
   poll_closest(L);
   poll_store(L, kAoClosestTest, 0.0f);
@@ -332,7 +332,7 @@ __global__ void k_ao_begin(AoLaunch L, uint32_t n, uint32_t nzero) {
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < nzero) L.tcount[t] = t == 0 ? n : 0u;  // the camera rays queued for round 2
-  if (t == 0) *L.work = 0u;                        // for round 2's traversal
+  if (blockIdx.x == 0) clear_work(L.work, threadIdx.x);  // for round 2's traversal
   const uint32_t s = __float_as_uint(L.frame[23]);
   for (uint32_t g = 0; g < L.gr.n; g++) {
     const Group &G = L.gr.g[g];

@@ -686,7 +686,7 @@ int32_t rdrt_trace(rdrt_ctx *c, const rdrt_trace_args *a) {
   if (a->traversal == RDRT_TRAVERSAL_FAST && stack_entries_for(push) == 0)
     return fail(RDRT_ERR_CAPACITY, "BVH too deep for the fast traversal stack (use RDRT_TRAVERSAL_REFERENCE)");
   if (c->tune.persist) {
-    RDRT_HIP(c->trace_work.reserve(4));
+    RDRT_HIP(c->trace_work.reserve(kWorkWords * 4));
     p.work = (uint32_t *)c->trace_work.ptr;
   }
   const bool cull = c->tune.cull && a->traversal == RDRT_TRAVERSAL_FAST;
@@ -776,7 +776,7 @@ int32_t rdrt_autotune(rdrt_ctx *c, const rdrt_trace_args *a, uint32_t reps, rdrt
   p.flags = a->flags;
   p.cull_mask = a->cull_mask;
   p.tlas_idx = a->tlas_idx;
-  RDRT_HIP(c->trace_work.reserve(4));
+  RDRT_HIP(c->trace_work.reserve(kWorkWords * 4));
   p.work = (uint32_t *)c->trace_work.ptr;
   CullScratch cs{};
   rc = cull_scratch(c, a->n, cs);
@@ -786,7 +786,7 @@ int32_t rdrt_autotune(rdrt_ctx *c, const rdrt_trace_args *a, uint32_t reps, rdrt
   float chosen_ms = -1.0f;
   for (uint32_t block : {64u, 128u, 256u})
     for (uint32_t lds : {8u, 16u})
-      for (uint32_t waves : {0u, 6u, 8u})
+      for (uint32_t waves : {0u, 6u})
         for (uint32_t shape = 0; shape < 12; shape++) {
           TraceTune t;
           t.block = block;

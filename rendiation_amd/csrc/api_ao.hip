@@ -117,7 +117,7 @@ int32_t reserve_ao(rdrt_ctx *c, uint32_t cap) {
   RDRT_HIP(s.tq.reserve((size_t)2 * ntrace * 4));
   RDRT_HIP(s.counts.reserve(8 * 4));
   RDRT_HIP(s.frame.reserve(kAoFrameWords * sizeof(float)));
-  RDRT_HIP(s.work.reserve(4));
+  RDRT_HIP(s.work.reserve(kWorkWords * 4));
   s.capacity = cap;
   return RDRT_OK;
 }
@@ -343,7 +343,7 @@ int32_t rdrt_ao_autotune(rdrt_ctx *c, const rdrt_ao_params *prm, void *accum, ui
   std::vector<std::pair<float, TraceTune>> timed;
   for (uint32_t block : {64u, 128u, 256u})
     for (uint32_t lds : {8u, 16u})
-      for (uint32_t waves : {0u, 6u, 8u})
+      for (uint32_t waves : {0u, 6u})
         for (uint32_t shape = 0; shape < 18 && rc == RDRT_OK; shape++) {
           TraceTune t;
           t.block = block;

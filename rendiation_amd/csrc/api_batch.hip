@@ -144,7 +144,7 @@ int32_t rdrt_trace_batched(rdrt_ctx *c, const rdrt_batch_params *a) {
   const size_t nblk = (n + kSpawnBlock - 1) / kSpawnBlock;
   RDRT_HIP(s.tmp.reserve(nblk * kSpawnBlock * 4));
   RDRT_HIP(s.blk.reserve(2 * nblk * 4));
-  RDRT_HIP(s.work.reserve(4));
+  RDRT_HIP(s.work.reserve(kWorkWords * 4));
   hipStream_t st = c->work_stream;
   s.rounds = pl.rounds;
   s.nscenes = pl.nscenes;
@@ -244,7 +244,7 @@ int32_t rdrt_batch_autotune(rdrt_ctx *c, const rdrt_batch_params *a, uint32_t re
   float chosen_ms = -1.0f;
   for (uint32_t block : {64u, 128u, 256u})
     for (uint32_t lds : {8u, 16u})
-      for (uint32_t waves : {0u, 6u, 8u})
+      for (uint32_t waves : {0u, 6u})
         for (uint32_t shape = 0; shape < 6 && rc == RDRT_OK; shape++) {
           TraceTune t;
           t.block = block;

@@ -117,7 +117,7 @@ int32_t reserve_pipeline(rdrt_pipeline *p, uint32_t cap) {
     S.call = carve<rdrt_trace_call>(p, n, e);
   }
   if (e != hipSuccess) return fail(RDRT_ERR_OUT_OF_MEMORY, std::string("pipeline buffers: ") + hipGetErrorString(e));
-  RDRT_HIP(p->work.reserve(4));
+  RDRT_HIP(p->work.reserve(kWorkWords * 4));
   p->capacity = cap;
   return RDRT_OK;
 }

@@ -259,7 +259,7 @@ int32_t rdrt_pt_render(rdrt_ctx *c, const rdrt_pt_params *prm, float *radiance) 
   L.blk = (uint32_t *)s.blk.ptr;
   L.blk_stride = (npaths + kPtBlock - 1) / kPtBlock;
   L.status = c->status;
-  RDRT_HIP(s.work.reserve(8));
+  RDRT_HIP(s.work.reserve((kWorkWords + 1) * 4));
   L.work = (uint32_t *)s.work.ptr;
   L.out = radiance;
   if (prm->record) {
@@ -394,7 +394,7 @@ int32_t rdrt_pt_autotune(rdrt_ctx *c, const rdrt_pt_params *prm, float *radiance
   };
   for (uint32_t block : {64u, 128u, 256u})
     for (uint32_t lds : {8u, 16u})
-      for (uint32_t waves : {0u, 6u, 8u})
+      for (uint32_t waves : {0u, 6u})
         for (uint32_t shape = 0; shape < 18 && rc == RDRT_OK; shape++) {
           TraceTune t;
           t.block = block;

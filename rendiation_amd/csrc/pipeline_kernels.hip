@@ -41,10 +41,10 @@ __global__ void k_pipe_trace_pre(PipeLaunch L) {
   uint32_t *cnt = L.tcount + L.qpar;
   // the other parity's count (used by the previous round, all of whose
   // launches have finished) starts the next round at zero, and so does the
-  // work counter of the traversal that follows
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    L.tcount[L.qpar ^ 1u] = 0u;
-    *L.work = 0u;
+  // work counters of the traversal that follows
+  if (blockIdx.x == 0) {
+    clear_work(L.work, threadIdx.x);
+    if (threadIdx.x == 0) L.tcount[L.qpar ^ 1u] = 0u;
   }
   tg::begin_phase(T);
   tg::refill_empty(T);  // trace slots are taken and freed only by stage polls

@@ -46,7 +46,7 @@ struct PtLaunch {
   uint32_t *tmp_a, *tmp_b, *blk;
   uint32_t blk_stride;
   uint32_t *status;
-  uint32_t *work;  // [0]: work counter of persistent traversal launches; [1]: of the tail kernel
+  uint32_t *work;  // counters of persistent traversal launches (kWorkWords), then the tail kernel's
   // tail: from bounce tail_b0 (>= 1) on, the tail kernel finishes every path
   // (0 = per-bounce launches throughout); tflags[path]: what shade(tail_b0)
   // left the path (bit 0: a shadow ray, bit 1: an extension ray)

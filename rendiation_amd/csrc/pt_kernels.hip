@@ -40,13 +40,18 @@ using compact::k_scatter2;
 using compact::kScanThreads;
 using namespace pts;
 
+__device__ __forceinline__ void clear_work_and_tail(const PtLaunch &P) {
+  clear_work(P.work, threadIdx.x);
+  if (threadIdx.x == 0) P.work[kWorkWords] = 0u;
+}
+
 __global__ void k_pt_begin(PtLaunch P) {
   const uint32_t nc = 2 * P.max_bounces + 3;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += gridDim.x * blockDim.x)
     P.counts[i] = i == 0 ? P.npaths : 0u;
   // the work counters of the persistent traversal and of the tail kernel
   // start at zero (so their launches need no clearing launch)
-  if (blockIdx.x == 0 && threadIdx.x < 2) P.work[threadIdx.x] = 0u;
+  if (blockIdx.x == 0) clear_work_and_tail(P);
 }
 
 // ray generation (ray_gen.rs:89-107 + camera.rs:66-99)
@@ -79,7 +84,7 @@ __global__ __launch_bounds__(B) void k_pt_shade(PtLaunch P, uint32_t b) {
   const uint32_t bid = blockIdx.x;
   // between the traversal of bounce b and the next one: the work counters of
   // the persistent traversal and the tail kernel start that one at zero
-  if (bid == 0 && threadIdx.x < 2) P.work[threadIdx.x] = 0u;
+  if (bid == 0) clear_work_and_tail(P);
   const uint32_t count_in = min(P.counts[b], P.npaths);
   const uint32_t nblocks = (count_in + B - 1) / B;
   if (bid >= nblocks) return;  // whole block
@@ -464,7 +469,7 @@ hipError_t enqueue_pt_frame(const PtLaunch &P, const TraceParams &scene, uint32_
       pe.queue = ps.queue = nullptr;
       pe.count = ps.count = nullptr;
       if (diag && diag->ev_begin) (void)hipEventRecord(diag->ev_begin[launch], st);
-      e = launch_pt_tail(P, pe, ps, push_depth, tune, st);  // work[1] zeroed by k_pt_shade(b)
+      e = launch_pt_tail(P, pe, ps, push_depth, tune, st);  // its counter cleared by k_pt_shade(b)
       if (diag && diag->ev_end) (void)hipEventRecord(diag->ev_end[launch], st);
       launch++;
       if (e != hipSuccess) return e;
@@ -519,6 +524,7 @@ hipError_t enqueue_pt_replay(const PtLaunch &P, const TraceParams &scene, uint32
     tp.cull_mask = 0xffffffffu;
     tp.tlas_idx = 0;
     tp.work = P.work;
+    tp.work_zeroed = 1u;  // by k_pt_begin / k_pt_shade
     e = launch_trace(tp, RDRT_TRAVERSAL_FAST, push_depth, tune, st);
     if (e != hipSuccess) return e;
     if (b == P.max_bounces) break;  // the last vertex adds no geometry term

@@ -35,14 +35,14 @@ constexpr uint32_t kTailBlock = 128;
 template <int K, int S, int LAYOUT>
 __global__ __launch_bounds__(kTailBlock) void k_pt_tail(PtLaunch P, TraceParams pe, TraceParams ps) {
   constexpr int B = (int)kTailBlock;
-  __shared__ uint32_t lds[K * B];
+  __shared__ uint32_t lds[LaneStack<K, S, B>::kRows * B];
   const uint32_t b0 = P.tail_b0;
   const uint32_t glane = threadIdx.x & (kCoopLanes - 1u);
   const uint32_t leader = __lane_id() & ~(kCoopLanes - 1u);
   const uint32_t nitems = min(P.counts[b0], P.npaths);
   const uint32_t *qin = (b0 & 1u) ? P.qb : P.qa;  // the queue shade(b0) read
   uint32_t *stk = lds + threadIdx.x;
-  uint32_t *next = P.work + 1;
+  uint32_t *next = P.work + kWorkWords;
   for (;;) {
     uint32_t item = 0;
     if (glane == 0) item = atomicAdd(next, 1u);

@@ -12,15 +12,27 @@
 //    hit/miss links (traverse_cpu.rs:283-319) in the reference order, with the
 //    reference's per-test arithmetic; its hits and visit counters equal the
 //    oracle's bit for bit.
-//  * k_trace_fast walks the 64-byte child-pair layout front to back with a
-//    per-lane stack in LDS (column layout [entry][lane]: each lane owns one
-//    bank at every depth, so stack traffic is conflict-free) and tests
-//    triangles from 64-byte pre-pass records.  The box and triangle
-//    arithmetic is the reference's, so t, u, v are bit-identical; only the
-//    visit order differs, which can change the winner among hits with equal t.
+//  * The fast kernels walk child-pair or child-quad layouts of a tree of
+//    their own front to back, with a per-lane stack in LDS (column layout
+//    [entry][lane]: each lane owns one bank at every depth, so stack traffic
+//    is conflict-free), and test triangles from 64-byte pre-pass records with
+//    the reference's arithmetic, so t, u, v are bit-identical.  Their node
+//    tests are fused multiply-adds widened by their rounding error: they may
+//    pass a box that the reference's test fails, never the other way round.
+//    Only the visit order differs, which can change the winner among hits with
+//    equal t.
+//
+//    What bounded these kernels was idle lanes: with every lane doing whatever
+//    it was at, 9 (1M rays in 100k triangles) to 15 (height field, first
+//    bounce) of 64 lanes worked per vector instruction.  trace_wave gives the
+//    wave one kind of work at a time and refills it: 19 to 30 lanes.  With the
+//    node tests in fewer instructions, no round trip to memory behind them and
+//    a work counter per XCD, 1M rays went from 0.487 to 0.337 ms, the 1080p
+//    frame from 2.39 to 1.85 ms, a height-field step of 16 views from 24.7 to
+//    20.8 ms, a batch of 16 scenes from 4.33 to 2.31 ms.
 //
 // Compiled with -ffp-contract=off and IEEE division/sqrt: one rounding per
-// operation, as in the reference.
+// operation, as in the reference, but for the node tests.
 #ifndef RDRT_TRACE_DEVICE_H
 #define RDRT_TRACE_DEVICE_H
 
@@ -221,246 +233,494 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t i, uint32_t used) {
   return xcd < rem ? xcd * (per + 1u) + local : rem * (per + 1u) + (xcd - rem) * per + local;
 }
 
-// Inner-node steps of the fast traversal.  Each tests the children of node
-// `ref`; when some are hit it sets ref to the nearest, pushes the others
-// (farthest first, so they pop near to far) and returns true.
-template <class Push>
-__device__ __forceinline__ bool step_pair(const PairNode *nodes, uint32_t &ref, F3 o, F3 inv_d, float tmin, float tmax,
-                                          Push &&push) {
-  const float4 *q = reinterpret_cast<const float4 *>(nodes + ref);
+// Inner-node tests of the fast traversal: the children of one node that the
+// ray meets, in `r[0 .. n)`, farthest first (what follows r[n - 1] is
+// undefined).
+struct Kids {
+  uint32_t n, r[4];
+};
+
+// A ray as the node tests take it: per axis 1 / dir and the constants of
+// t = plane * inv + bias for the near and the far planes.  The fused form
+// takes half the instructions of (plane - o) * inv; its rounding error against
+// that form is that of o * inv, at most 2^-23 |o * inv|, which the biases
+// move outwards, so a node test may pass a box that the exact test fails,
+// never the other way round.  |inv| is bounded (2^60), so that an axis-parallel
+// ray gets large finite distances and no NaN on that axis.
+struct RayBox {
+  F3 inv, nb, fb;
+};
+__device__ __forceinline__ void ray_box_axis(float o, float inv, float &iv, float &nb, float &fb) {
+  constexpr float kMost = 1.152921504606846976e18f, kErr = 2.384185791015625e-7f;  // 2^60, 2^-22
+  iv = fminf(fmaxf(inv, -kMost), kMost);
+  const float c = -(o * iv), e = fabsf(c) * kErr;
+  nb = c - e;
+  fb = c + e;
+}
+__device__ __forceinline__ RayBox ray_box(F3 o, F3 inv) {
+  RayBox r;
+  ray_box_axis(o.x, inv.x, r.inv.x, r.nb.x, r.fb.x);
+  ray_box_axis(o.y, inv.y, r.inv.y, r.nb.y, r.fb.y);
+  ray_box_axis(o.z, inv.z, r.inv.z, r.nb.z, r.fb.z);
+  return r;
+}
+__device__ __forceinline__ bool negative(float v) { return (__float_as_uint(v) & 0x80000000u) != 0u; }
+
+// Near and far planes (already chosen by the direction's sign) of one box.
+__device__ __forceinline__ bool box_hit(const RayBox &r, float tmin, float tmax, float nx, float ny, float nz, float fx,
+                                        float fy, float fz, float &tnear) {
+  const float tn = fmaxf(fmaxf(__builtin_fmaf(nx, r.inv.x, r.nb.x), __builtin_fmaf(ny, r.inv.y, r.nb.y)),
+                         __builtin_fmaf(nz, r.inv.z, r.nb.z));
+  const float tf = fminf(fminf(__builtin_fmaf(fx, r.inv.x, r.fb.x), __builtin_fmaf(fy, r.inv.y, r.fb.y)),
+                         __builtin_fmaf(fz, r.inv.z, r.fb.z));
+  tnear = tn;
+  return tn <= tf && tmin < tf && tn < tmax;
+}
+
+__device__ __forceinline__ Kids kids_pair(const PairNode *node, const RayBox &r, float tmin, float tmax) {
+  const float4 *q = reinterpret_cast<const float4 *>(node);
   const float4 a = q[0], b = q[1], c = q[2], d = q[3];
+  const bool sx = negative(r.inv.x), sy = negative(r.inv.y), sz = negative(r.inv.z);
   float tl, tr;
-  const bool hl = slab(o, inv_d, tmin, tmax, a.x, a.y, a.z, b.x, b.y, b.z, tl);
-  const bool hr = slab(o, inv_d, tmin, tmax, c.x, c.y, c.z, d.x, d.y, d.z, tr);
+  const bool hl = box_hit(r, tmin, tmax, sx ? b.x : a.x, sy ? b.y : a.y, sz ? b.z : a.z, sx ? a.x : b.x,
+                          sy ? a.y : b.y, sz ? a.z : b.z, tl);
+  const bool hr = box_hit(r, tmin, tmax, sx ? d.x : c.x, sy ? d.y : c.y, sz ? d.z : c.z, sx ? c.x : d.x,
+                          sy ? c.y : d.y, sz ? c.z : d.z, tr);
   const uint32_t lref = __float_as_uint(a.w), rref = __float_as_uint(c.w);
-  if (hl && hr) {
-    const bool rfirst = tr < tl;
-    push(rfirst ? lref : rref);
-    ref = rfirst ? rref : lref;
-    return true;
-  }
-  if (hl || hr) {
-    ref = hl ? lref : rref;
-    return true;
-  }
-  return false;
+  const bool rlast = hr && (!hl || tr < tl);  // the right child is the nearest hit
+  Kids k;
+  k.n = (uint32_t)hl + (uint32_t)hr;
+  const uint32_t near_ref = rlast ? rref : lref, far_ref = rlast ? lref : rref;
+  k.r[0] = k.n == 2u ? far_ref : near_ref;
+  k.r[1] = near_ref;
+  k.r[2] = k.r[3] = 0u;
+  return k;
 }
 
-// Sort key of one quad child: its entry distance when hit (never NaN, always
-// below +inf: a hit's entry lies below tmax), +inf when missed or unused.
-__device__ __forceinline__ float quad_key(bool hit, float tnear) {
-  return hit ? fmaxf(tnear, -3.402823466e38f) : __builtin_inff();
+// Sort key of one quad child: a double whose high word is the entry distance
+// and whose low word is the child's ref, 0 when missed.  Distances are
+// clamped to at least 2^-100, so every hit is a positive normal double (its
+// float bits are below those of infinity) and the order of the doubles is the
+// order of the distances.
+__device__ __forceinline__ double quad_key(bool hit, float tnear, uint32_t ref) {
+  const uint32_t hi = hit ? __float_as_uint(fmaxf(tnear, 7.88860905e-31f)) : 0u;
+  return __hiloint2double((int)hi, (int)ref);
 }
-__device__ __forceinline__ void order2(float &ka, uint32_t &ra, float &kb, uint32_t &rb) {
-  const bool sw = kb < ka;
-  const float k = sw ? kb : ka;
-  const uint32_t r = sw ? rb : ra;
-  kb = sw ? ka : kb;
-  rb = sw ? ra : rb;
-  ka = k;
-  ra = r;
+// One compare-exchange in two instructions (fmin / fmax on values that the
+// compiler cannot prove to be no signaling NaN take four).
+__device__ __forceinline__ void order2(double &a, double &b) {
+  double hi, lo;
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+  a = hi;
+  b = lo;
 }
-
-template <class Push>
-__device__ __forceinline__ bool step_quad(const QuadNode *nodes, uint32_t &ref, F3 o, F3 inv_d, float tmin, float tmax,
-                                          Push &&push) {
-  const float4 *q = reinterpret_cast<const float4 *>(nodes + ref);
-  const float4 x0 = q[0], x1 = q[1], y0 = q[2], y1 = q[3], z0 = q[4], z1 = q[5];
-  const uint4 rf = *reinterpret_cast<const uint4 *>(q + 6);
-  float t0, t1, t2, t3;
-  const bool h0 = slab(o, inv_d, tmin, tmax, x0.x, y0.x, z0.x, x1.x, y1.x, z1.x, t0);
-  const bool h1 = slab(o, inv_d, tmin, tmax, x0.y, y0.y, z0.y, x1.y, y1.y, z1.y, t1);  // slots 0, 1 always used
-  const bool h2 = slab(o, inv_d, tmin, tmax, x0.z, y0.z, z0.z, x1.z, y1.z, z1.z, t2) && rf.z != kInvalid;
-  const bool h3 = slab(o, inv_d, tmin, tmax, x0.w, y0.w, z0.w, x1.w, y1.w, z1.w, t3) && rf.w != kInvalid;
-  const uint32_t n = (uint32_t)h0 + (uint32_t)h1 + (uint32_t)h2 + (uint32_t)h3;
-  if (n == 0) return false;
-  float k0 = quad_key(h0, t0), k1 = quad_key(h1, t1), k2 = quad_key(h2, t2), k3 = quad_key(h3, t3);
-  uint32_t r0 = rf.x, r1 = rf.y, r2 = rf.z, r3 = rf.w;
-  // sorting network of four: hits ascend by entry distance, misses last
-  order2(k0, r0, k1, r1);
-  order2(k2, r2, k3, r3);
-  order2(k0, r0, k2, r2);
-  order2(k1, r1, k3, r3);
-  order2(k1, r1, k2, r2);
-  if (n > 3) push(r3);
-  if (n > 2) push(r2);
-  if (n > 1) push(r1);
-  ref = r0;
-  return true;
+__device__ __forceinline__ Kids sort_kids(const bool h[4], const float t[4], uint4 rf) {
+  double k0 = quad_key(h[0], t[0], rf.x), k1 = quad_key(h[1], t[1], rf.y), k2 = quad_key(h[2], t[2], rf.z),
+         k3 = quad_key(h[3], t[3], rf.w);
+  // sorting network of four: hits descend by entry distance, misses last
+  order2(k0, k1);
+  order2(k2, k3);
+  order2(k0, k2);
+  order2(k1, k3);
+  order2(k1, k2);
+  Kids k;
+  k.n = (uint32_t)h[0] + (uint32_t)h[1] + (uint32_t)h[2] + (uint32_t)h[3];
+  k.r[0] = (uint32_t)__double2loint(k0);
+  k.r[1] = (uint32_t)__double2loint(k1);
+  k.r[2] = (uint32_t)__double2loint(k2);
+  k.r[3] = (uint32_t)__double2loint(k3);
+  return k;
 }
 
-// Byte c of a quantized node word, decoded: corner + q * step (q * step is
-// exact, the sum rounds once, as on the host that chose q).
-__device__ __forceinline__ float dequant(float corner, uint32_t word, int c, float step) {
-  return corner + (float)((word >> (8 * c)) & 0xffu) * step;
+__device__ __forceinline__ Kids kids_quad(const QuadNode *node, const RayBox &r, float tmin, float tmax) {
+  // the rows of the near and the far planes of an axis swap with the
+  // direction's sign: 16 bytes apart, so the loads pick them
+  const char *q = reinterpret_cast<const char *>(node);
+  const uint32_t sx = (__float_as_uint(r.inv.x) >> 27) & 16u, sy = (__float_as_uint(r.inv.y) >> 27) & 16u,
+                 sz = (__float_as_uint(r.inv.z) >> 27) & 16u;
+  const float4 xn = *reinterpret_cast<const float4 *>(q + sx), xf = *reinterpret_cast<const float4 *>(q + (sx ^ 16u));
+  const float4 yn = *reinterpret_cast<const float4 *>(q + 32 + sy),
+               yf = *reinterpret_cast<const float4 *>(q + 32 + (sy ^ 16u));
+  const float4 zn = *reinterpret_cast<const float4 *>(q + 64 + sz),
+               zf = *reinterpret_cast<const float4 *>(q + 64 + (sz ^ 16u));
+  const uint4 rf = *reinterpret_cast<const uint4 *>(q + 96);
+  float t[4];
+  bool h[4];
+  h[0] = box_hit(r, tmin, tmax, xn.x, yn.x, zn.x, xf.x, yf.x, zf.x, t[0]);
+  h[1] = box_hit(r, tmin, tmax, xn.y, yn.y, zn.y, xf.y, yf.y, zf.y, t[1]);  // slots 0, 1 always used
+  h[2] = box_hit(r, tmin, tmax, xn.z, yn.z, zn.z, xf.z, yf.z, zf.z, t[2]) && rf.z != kInvalid;
+  h[3] = box_hit(r, tmin, tmax, xn.w, yn.w, zn.w, xf.w, yf.w, zf.w, t[3]) && rf.w != kInvalid;
+  return sort_kids(h, t, rf);
 }
 
-template <class Push>
-__device__ __forceinline__ bool step_qquad(const QuadNodeQ *nodes, uint32_t &ref, F3 o, F3 inv_d, float tmin,
-                                           float tmax, Push &&push) {
-  const float4 *q = reinterpret_cast<const float4 *>(nodes + ref);
+// Quantized planes: corner + q * step, so t = q * (step * inv) + (corner *
+// inv + bias): two instructions per plane (byte to float, fused multiply-add).
+// The rounding of step * inv, at most 255 * 2^-24 of it, moves the bias
+// outwards too.
+__device__ __forceinline__ float quant_t(uint32_t word, int c, float step, float base) {
+  return __builtin_fmaf((float)((word >> (8 * c)) & 0xffu), step, base);
+}
+
+__device__ __forceinline__ Kids kids_qquad(const QuadNodeQ *node, const RayBox &r, float tmin, float tmax) {
+  const float4 *q = reinterpret_cast<const float4 *>(node);
   const float4 a = q[0];                                  // corner, x step
   const uint4 rf = *reinterpret_cast<const uint4 *>(q + 1);
   const uint4 xy = *reinterpret_cast<const uint4 *>(q + 2);  // lox, hix, loy, hiy
   const float4 zs = q[3];                                 // loz, hiz (bits), y step, z step
   const uint32_t loz = __float_as_uint(zs.x), hiz = __float_as_uint(zs.y);
+  const bool sx = negative(r.inv.x), sy = negative(r.inv.y), sz = negative(r.inv.z);
+  const uint32_t nx = sx ? xy.y : xy.x, fx = sx ? xy.x : xy.y, ny = sy ? xy.w : xy.z, fy = sy ? xy.z : xy.w,
+                 nz = sz ? hiz : loz, fz = sz ? loz : hiz;
+  constexpr float kErr = 6.103515625e-5f;  // 2^-14 > 255 * 2^-23
+  const float ax = a.w * r.inv.x, ay = zs.z * r.inv.y, az = zs.w * r.inv.z;
+  const float bnx = __builtin_fmaf(fabsf(ax), -kErr, __builtin_fmaf(a.x, r.inv.x, r.nb.x)),
+              bny = __builtin_fmaf(fabsf(ay), -kErr, __builtin_fmaf(a.y, r.inv.y, r.nb.y)),
+              bnz = __builtin_fmaf(fabsf(az), -kErr, __builtin_fmaf(a.z, r.inv.z, r.nb.z)),
+              bfx = __builtin_fmaf(fabsf(ax), kErr, __builtin_fmaf(a.x, r.inv.x, r.fb.x)),
+              bfy = __builtin_fmaf(fabsf(ay), kErr, __builtin_fmaf(a.y, r.inv.y, r.fb.y)),
+              bfz = __builtin_fmaf(fabsf(az), kErr, __builtin_fmaf(a.z, r.inv.z, r.fb.z));
   float t[4];
   bool h[4];
 #pragma unroll
-  for (int c = 0; c < 4; c++)
-    h[c] = slab(o, inv_d, tmin, tmax, dequant(a.x, xy.x, c, a.w), dequant(a.y, xy.z, c, zs.z),
-                dequant(a.z, loz, c, zs.w), dequant(a.x, xy.y, c, a.w), dequant(a.y, xy.w, c, zs.z),
-                dequant(a.z, hiz, c, zs.w), t[c]);
+  for (int c = 0; c < 4; c++) {
+    const float tn = fmaxf(fmaxf(quant_t(nx, c, ax, bnx), quant_t(ny, c, ay, bny)), quant_t(nz, c, az, bnz));
+    const float tf = fminf(fminf(quant_t(fx, c, ax, bfx), quant_t(fy, c, ay, bfy)), quant_t(fz, c, az, bfz));
+    t[c] = tn;
+    h[c] = tn <= tf && tmin < tf && tn < tmax;
+  }
   h[2] = h[2] && rf.z != kInvalid;  // slots 0, 1 always used
   h[3] = h[3] && rf.w != kInvalid;
-  const uint32_t n = (uint32_t)h[0] + (uint32_t)h[1] + (uint32_t)h[2] + (uint32_t)h[3];
-  if (n == 0) return false;
-  float k0 = quad_key(h[0], t[0]), k1 = quad_key(h[1], t[1]), k2 = quad_key(h[2], t[2]), k3 = quad_key(h[3], t[3]);
-  uint32_t r0 = rf.x, r1 = rf.y, r2 = rf.z, r3 = rf.w;
-  order2(k0, r0, k1, r1);
-  order2(k2, r2, k3, r3);
-  order2(k0, r0, k2, r2);
-  order2(k1, r1, k3, r3);
-  order2(k1, r1, k2, r2);
-  if (n > 3) push(r3);
-  if (n > 2) push(r2);
-  if (n > 1) push(r1);
-  ref = r0;
-  return true;
+  return sort_kids(h, t, rf);
 }
 
-// ------------------------------------------------------------------------
-// Fast kernel: front-to-back child-pair traversal.  Stack: the first K
-// entries of each lane live in LDS (column layout), deeper ones (rare) in
-// the lane's private memory; S bounds the total.
-// ------------------------------------------------------------------------
-template <int K, int S, int B, bool CNT, int LAYOUT>
-__device__ __forceinline__ void trace_fast_one(const TraceParams &p, uint32_t rid, uint32_t *stk) {
-  uint32_t spill[S > K ? S - K : 1];
-  auto push = [&](uint32_t &sp, uint32_t v) {
-    if (sp < (uint32_t)K) stk[sp * B] = v;
-    else if (sp < (uint32_t)S) spill[sp - K] = v;
-    else {
-      atomicOr(p.status, 1u);  // unreachable when S covers the built depth
-      return;
+template <int LAYOUT>
+__device__ __forceinline__ Kids test_kids(const TraceParams &p, bool world, uint32_t ref, const RayBox &r, float tmin,
+                                          float tmax) {
+  if constexpr (LAYOUT == 2) return kids_qquad((world ? p.tlas_qquads : p.tri_qquads) + ref, r, tmin, tmax);
+  else if constexpr (LAYOUT == 1) return kids_quad((world ? p.tlas_quads : p.tri_quads) + ref, r, tmin, tmax);
+  else return kids_pair((world ? p.tlas_pairs : p.tri_pairs) + ref, r, tmin, tmax);
+}
+
+// A lane's traversal stack: the first R entries in LDS (column layout:
+// entry i of the lane at lds[i * B], its own bank at every depth), deeper
+// ones (rare) in the lane's private memory.  It holds up to S node refs and
+// two end marks.  A step writes its (up to) three farther children at the
+// top without asking how many there are and reads the entry below before its
+// node arrives, so neither branches nor a second round trip to memory follow
+// the box tests.
+template <int K, int S, int B>
+struct LaneStack {
+  static constexpr uint32_t R = K + 4, N = S + 2, kSpill = N > R ? N - R : 1, kRows = R + 6;
+  uint32_t *lds;
+  // kSpill words of private memory: an array of its own (inside, it would keep sp in memory too) and volatile (else the
+  // compiler turns it into registers that it indexes in loops)
+  volatile uint32_t *spill;
+  uint32_t *status;
+  uint32_t sp;
+
+  // the object-space ray of the lane's instance, for the triangle tests, in
+  // the six LDS rows above the stack (the node tests need only the RayBox)
+  __device__ __forceinline__ void set_ray(F3 o, F3 d) {
+    float *q = reinterpret_cast<float *>(lds + R * B);
+    q[0] = o.x, q[B] = o.y, q[2 * B] = o.z, q[3 * B] = d.x, q[4 * B] = d.y, q[5 * B] = d.z;
+  }
+  __device__ __forceinline__ void get_ray(F3 &o, F3 &d) const {
+    const float *q = reinterpret_cast<const float *>(lds + R * B);
+    o = f3(q[0], q[B], q[2 * B]);
+    d = f3(q[3 * B], q[4 * B], q[5 * B]);
+  }
+  __device__ __forceinline__ bool deep() const { return sp + 3u > R; }
+  __device__ __forceinline__ uint32_t get(uint32_t i) const {
+    if (N <= R || i < R) return lds[i * B];
+    uint32_t v = spill[i - R];
+    asm volatile("" : "+v"(v));  // keeps the two loads apart: one load through a selected pointer would be a flat one
+    return v;
+  }
+  __device__ __forceinline__ void put(uint32_t i, uint32_t v) {
+    if (i < (N < R ? N : R)) lds[i * B] = v;
+    else if (i < N) spill[i - R] = v;
+    else atomicOr(status, 1u);  // unreachable when S covers the built depth
+  }
+  __device__ __forceinline__ void push(uint32_t v) {
+    put(sp, v);
+    if (sp < N) sp++;
+  }
+  __device__ __forceinline__ uint32_t pop() { return get(--sp); }
+
+  // The step of a lane at an inner node: kids() tests the node; returns the
+  // nearest child hit, or the top of the stack when none is.
+  template <int LAYOUT, class F>
+  __device__ __forceinline__ uint32_t step(F &&kids) {
+    const bool slow = __ballot(deep()) != 0ull;  // wave-uniform, rare
+    const uint32_t top = slow ? get(sp - 1u) : lds[(sp - 1u) * B];
+    const Kids k = kids();
+    if (slow) {
+      for (uint32_t j = 0; j + 1u < k.n; j++) put(sp + j, j == 0u ? k.r[0] : j == 1u ? k.r[1] : k.r[2]);
+    } else {
+      uint32_t *at = lds + sp * B;
+      at[0] = k.r[0];
+      if constexpr (LAYOUT != 0) {
+        at[B] = k.r[1];
+        at[2 * B] = k.r[2];
+      }
     }
-    sp++;
-  };
-  auto pop = [&](uint32_t &sp) -> uint32_t {
-    sp--;
-    return sp < (uint32_t)K ? stk[sp * B] : spill[sp - K];
-  };
+    sp = min(sp + k.n - 1u, N);
+    uint32_t r = k.n == 1u ? k.r[0] : top;
+    r = k.n == 2u ? k.r[1] : r;
+    if constexpr (LAYOUT != 0) {
+      r = k.n == 3u ? k.r[2] : r;
+      r = k.n == 4u ? k.r[3] : r;
+    }
+    return r;
+  }
+};
 
-  RayIn r = load_ray(p, rid);
-  float far_ = r.tmax;
-  Best best;
+// ------------------------------------------------------------------------
+// Fast kernel: front-to-back traversal, one ray per lane, one kind of work
+// per wave step.
+//
+// A lane is at an inner node, at a leaf of triangles, or at the TLAS (a leaf
+// of instances, or a BLAS it has finished).  Each wave step does the work that
+// enough lanes wait for, the others keep their place: an inner step serves
+// TLAS and BLAS alike (the lane's current ray is the world or the object
+// ray), a leaf step tests all triangles of the leaf.  A loop in which every
+// lane does whatever it is at runs all three bodies for a few lanes each.
+// ------------------------------------------------------------------------
+constexpr uint32_t kRefExit = 0x7ffffff0u;  // the lane's BLAS is exhausted
+constexpr uint32_t kRefDone = 0x7ffffff1u;  // the lane's ray is finished (or it has none)
+// lane status bits
+constexpr uint32_t kStOpaque = 1u, kStCull = 2u, kStCullBack = 4u, kStEnd = 8u, kStSecond = 16u, kStBack = 32u,
+                   kStWorld = 64u;
+constexpr uint32_t kStMoreShift = 8;  // instances of the TLAS leaf still to visit
+
+__device__ __forceinline__ uint32_t wave_rank(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// Lanes of the wave for which v holds, as a scalar.
+__device__ __forceinline__ uint32_t wave_count(bool v) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)__popcll(__ballot(v)));
+}
+
+// Traces the slots [next, end) of the launch and every chunk that more(next,
+// end) gets after them (false: no more), refilling the wave when kRefill
+// lanes are idle.  Slots below n0 belong to the first segment.
+constexpr uint32_t kRefill = 32;
+// Inner steps go on while 1 / kKeep of the busy lanes want them.  Fewer lanes
+// waste vector instructions, more hold back the leaves whose hits shorten the
+// rays (2, 3, 4, 8: 366, 377, 431, 483 us for 1M rays in 100k triangles, but
+// 4.42, 4.15, 4.51, 4.50 ms for a batch of 16 scenes, measured on an earlier
+// build of these kernels).
+constexpr uint32_t kKeep = 3;
+
+template <int K, int S, int B, bool CNT, int LAYOUT, class More>
+__device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, uint32_t next, uint32_t end,
+                                           uint32_t *lds, More &&more) {
+  volatile uint32_t spill[LaneStack<K, S, B>::kSpill];
+  LaneStack<K, S, B> stk{lds, spill, p.status, 1u};
+  RayBox box = {};                               // the current ray: world or object space
+  float near_ = 0.0f, far_ = 0.0f, s = 1.0f;     // range: [near_, far_ * s] in its space
+  uint32_t ref = kRefDone, rid = kInvalid, st = 0u, inst = 0u, geo = 0u;
+  uint32_t best_k = kInvalid, best_geo = 0u, best_inst = 0u;
+  float best_u = 0.0f, best_v = 0.0f;
   uint32_t cn = 0, ct = 0, ci = 0;
-  bool done = false;
+  bool last = false;  // no chunk is left
 
-  const TlasRoot *root = bound_root(p, r.tlas_idx);
-  F3 winv = recip(r.d);
-  float tn;
-  if (root && slab(r.o, winv, r.tmin, far_, root->mn[0], root->mn[1], root->mn[2], root->mx[0], root->mx[1],
-                   root->mx[2], tn)) {
-    uint32_t sp = 0;
-    uint32_t ref = LAYOUT ? p.tlas_quad_roots[root - p.tlas_roots] : root->root_ref;
-    auto push_tlas = [&](uint32_t v) { push(sp, v); };
-    for (;;) {
-      if (!(ref & kLeafBit)) {
-        if constexpr (LAYOUT == 2) {
-          if (step_qquad(p.tlas_qquads, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
-        } else if constexpr (LAYOUT == 1) {
-          if (step_quad(p.tlas_quads, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
-        } else {
-          if (step_pair(p.tlas_pairs, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
+  auto ray_of = [&]() {
+    TraceParams q = p;
+    if (st & kStSecond) {
+      q.rays = p.rays2;
+      q.flags = p.flags2;
+    }
+    return load_ray(q, rid);
+  };
+
+  for (;;) {
+    const uint32_t idle = wave_count(ref == kRefDone);
+    if (idle == 64u || (!last && idle >= kRefill)) {
+      if (ref == kRefDone && rid != kInvalid) {
+        Best best;
+        best.k = best_k;
+        best.geo = best_geo;
+        best.inst = best_inst;
+        best.t = far_;  // far shrinks to each accepted hit
+        best.u = best_u;
+        best.v = best_v;
+        best.back = (st & kStBack) != 0u;
+        TraceParams q = p;
+        if (st & kStSecond) {
+          q.hits = p.hits2;
+          q.hitx = p.hitx2;
+          q.counters = nullptr;
         }
-      } else {
-        const uint32_t i0 = (ref & ~kLeafBit) >> kLeafCountBits, i1 = i0 + (ref & kLeafMaxCount);
-        for (uint32_t i = i0; i < i1 && !done; i++) {
-          if constexpr (CNT) ci++;
-          const InstRec &in = p.insts[i];
-          float ti;
-          if (!slab(r.o, winv, r.tmin, far_, in.mn[0], in.mn[1], in.mn[2], in.mx[0], in.mx[1], in.mx[2], ti))
-            continue;
-          if ((r.mask & in.mask) == 0) continue;
-          const uint32_t fl = merge_flags(r.flags, in.flags);
-          if (fl & F_SKIP_TRIANGLES) continue;
-          F3 bo, bd;
-          float s;
-          object_ray(in.inv, r.o, r.d, bo, bd, s);
-          const F3 binv = recip(bd);
-          const float near_s = r.tmin * s;
-          bool ce, cb;
-          cull_triangle(fl, ce, cb);
-          for (uint32_t g = in.geo_begin; g < in.geo_end && !done; g++) {
-            const GeoRec &geo = p.geos[g];
-            if (!geometry_passes(fl, geo.flags)) continue;
-            const bool opq = geometry_opaque(fl, geo.flags);
-            float tg;
-            if (!slab(bo, binv, near_s, far_ * s, geo.mn[0], geo.mn[1], geo.mn[2], geo.mx[0], geo.mx[1],
-                      geo.mx[2], tg))
-              continue;
-            // BLAS traversal; its stack entries sit above the TLAS ones.
-            uint32_t bsp = sp;
-            uint32_t bref = LAYOUT ? geo.quad_root : geo.root_ref;
-            auto push_blas = [&](uint32_t v) { push(bsp, v); };
-            for (;;) {
-              if (!(bref & kLeafBit)) {
-                if constexpr (CNT) cn++;
-                const float fs = far_ * s;
-                if constexpr (LAYOUT == 2) {
-                  if (step_qquad(p.tri_qquads, bref, bo, binv, near_s, fs, push_blas)) continue;
-                } else if constexpr (LAYOUT == 1) {
-                  if (step_quad(p.tri_quads, bref, bo, binv, near_s, fs, push_blas)) continue;
-                } else {
-                  if (step_pair(p.tri_pairs, bref, bo, binv, near_s, fs, push_blas)) continue;
-                }
-              } else {
-                const uint32_t k0 = (bref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (bref & kLeafMaxCount);
-                for (uint32_t k = k0; k < k1; k++) {
-                  if constexpr (CNT) ct++;
-                  const float4 *q = reinterpret_cast<const float4 *>(p.tris + k);
-                  float4 a = q[0], b = q[1], c = q[2], d = q[3];
-                  float t, u, v;
-                  bool back;
-                  if (tri_core(bo, bd, near_s, far_ * s, f3(a.x, a.y, a.z), f3(b.x, b.y, b.z), f3(c.x, c.y, c.z),
-                               f3(d.x, d.y, d.z), a.w, b.w, c.w, d.w, ce, cb, t, u, v, back)) {
-                    uint32_t beh = opq ? RDRT_ANYHIT_ACCEPT : anyhit_behavior(p, false, p.tri_ids[k]);
-                    if (beh & RDRT_ANYHIT_ACCEPT) {
-                      far_ = t / s;
-                      best.k = k;
-                      best.geo = g;
-                      best.inst = i;
-                      best.u = u;
-                      best.v = v;
-                      best.back = back;
-                      if (fl & F_END_SEARCH) beh |= RDRT_ANYHIT_END_SEARCH;
-                    }
-                    if (beh & RDRT_ANYHIT_END_SEARCH) {
-                      done = true;
-                      break;
-                    }
-                  }
-                }
-                if (done) break;
-              }
-              if (bsp == sp) break;
-              bref = pop(bsp);
+        write_result(q, p.tri_ids, rid, best, cn, ct, ci);
+        rid = kInvalid;
+      }
+      if (next >= end) {
+        if (!last) last = !more(next, end);
+        if (last) {
+          if (idle == 64u) break;
+          continue;
+        }
+      }
+      const uint64_t m = __ballot(ref == kRefDone);
+      const uint32_t slot = next + wave_rank(m);
+      if (ref == kRefDone && slot < end) {
+        const bool second = slot >= n0;
+        st = kStWorld | (second ? kStSecond : 0u);
+        const uint32_t qs = second ? slot - n0 : slot;
+        const uint32_t *queue = second ? p.queue2 : p.queue;
+        rid = queue ? queue[qs] : qs;
+        if (rid < p.n) {  // a queue entry always names one of the n rays
+          const RayIn r = ray_of();
+          const F3 winv = recip(r.d);
+          box = ray_box(r.o, winv);
+          near_ = r.tmin;
+          far_ = r.tmax;
+          s = 1.0f;
+          best_k = kInvalid;
+          if constexpr (CNT) cn = ct = ci = 0u;
+          const TlasRoot *root = bound_root(p, r.tlas_idx);
+          float tn;
+          if (root && slab(r.o, winv, near_, far_, root->mn[0], root->mn[1], root->mn[2], root->mx[0], root->mx[1],
+                           root->mx[2], tn)) {
+            ref = LAYOUT ? p.tlas_quad_roots[root - p.tlas_roots] : root->root_ref;
+            stk.lds[0] = kRefDone;  // the end mark of the ray
+            stk.sp = 1u;
+          }
+        } else {
+          rid = kInvalid;
+        }
+      }
+      next = min(end, next + idle);
+      continue;
+    }
+    uint32_t a = wave_count(ref < kRefExit);
+    if (a * kKeep >= 64u - idle) {
+      do {
+        if (ref < kRefExit) {
+          const bool world = (st & kStWorld) != 0u;
+          if constexpr (CNT) cn += world ? 0u : 1u;
+          const float fs = far_ * s;
+          ref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, world, ref, box, near_, fs); });
+        }
+        a = wave_count(ref < kRefExit);
+      } while (a * kKeep >= 64u - idle);
+      continue;
+    }
+    const bool leaf = (ref & kLeafBit) != 0u, world = (st & kStWorld) != 0u;
+    if (wave_count(leaf && !world) >= wave_count(ref == kRefExit || (leaf && world))) {
+      if (leaf && !world) {
+        const uint32_t k0 = (ref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (ref & kLeafMaxCount);
+        F3 o, bd;
+        stk.get_ray(o, bd);
+        ref = stk.get(stk.sp - 1u);
+        for (uint32_t k = k0; k < k1; k++) {
+          if constexpr (CNT) ct++;
+          const float4 *q = reinterpret_cast<const float4 *>(p.tris + k);
+          const float4 ta = q[0], tb = q[1], tc = q[2], td = q[3];
+          float t, u, v;
+          bool back;
+          if (tri_core(o, bd, near_, far_ * s, f3(ta.x, ta.y, ta.z), f3(tb.x, tb.y, tb.z), f3(tc.x, tc.y, tc.z),
+                       f3(td.x, td.y, td.z), ta.w, tb.w, tc.w, td.w, (st & kStCull) != 0u, (st & kStCullBack) != 0u, t,
+                       u, v, back)) {
+            uint32_t beh = (st & kStOpaque) ? RDRT_ANYHIT_ACCEPT : anyhit_behavior(p, false, p.tri_ids[k]);
+            if (beh & RDRT_ANYHIT_ACCEPT) {
+              far_ = t / s;
+              best_k = k;
+              best_geo = geo;
+              best_inst = inst;
+              best_u = u;
+              best_v = v;
+              st = back ? st | kStBack : st & ~kStBack;
+              if (st & kStEnd) beh |= RDRT_ANYHIT_END_SEARCH;
+            }
+            if (beh & RDRT_ANYHIT_END_SEARCH) {
+              ref = kRefDone;
+              break;
             }
           }
-          // re-read the world ray instead of keeping it live through the BLAS loop
-          r = load_ray(p, rid);
-          winv = recip(r.d);
         }
-        if (done) break;
+        stk.sp--;
       }
-      if (sp == 0) break;
-      ref = pop(sp);
+    } else if (ref == kRefExit || (leaf && world)) {
+      // the next geometry of the lane's instance, or the next instance of its
+      // TLAS leaf, that the ray may hit; back to the TLAS when there is none
+      const RayIn r = ray_of();
+      const F3 winv = recip(r.d);
+      uint32_t left, g, gend, fl;
+      F3 o = r.o, inv = winv;  // the object ray of the instance
+      if (world) {
+        inst = ((ref & ~kLeafBit) >> kLeafCountBits) - 1u;
+        left = ref & kLeafMaxCount;
+        g = gend = fl = 0u;
+      } else {
+        left = st >> kStMoreShift;
+        const InstRec &in = p.insts[inst];
+        g = geo + 1u;
+        gend = in.geo_end;
+        fl = merge_flags(r.flags, in.flags);
+        if (g < gend) {
+          F3 bd;
+          stk.get_ray(o, bd);
+          inv = recip(bd);
+        }
+      }
+      for (;;) {
+        if (g < gend) {
+          const GeoRec &gr = p.geos[g];
+          float tg;
+          if (geometry_passes(fl, gr.flags) && slab(o, inv, near_, far_ * s, gr.mn[0], gr.mn[1], gr.mn[2], gr.mx[0],
+                                                    gr.mx[1], gr.mx[2], tg)) {
+            bool ce, cb;
+            cull_triangle(fl, ce, cb);
+            st = (st & (kStSecond | kStBack)) | (geometry_opaque(fl, gr.flags) ? kStOpaque : 0u) |
+                 (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) | ((fl & F_END_SEARCH) ? kStEnd : 0u) |
+                 (left << kStMoreShift);
+            geo = g;
+            box = ray_box(o, inv);
+            stk.push(kRefExit);  // the end mark of the BLAS, above the TLAS entries
+            ref = LAYOUT ? gr.quad_root : gr.root_ref;
+            break;
+          }
+          g++;
+          continue;
+        }
+        if (left == 0u) {
+          box = ray_box(r.o, winv);
+          near_ = r.tmin;
+          s = 1.0f;
+          st |= kStWorld;
+          ref = stk.pop();
+          break;
+        }
+        inst++;
+        left--;
+        if constexpr (CNT) ci++;
+        const InstRec &in = p.insts[inst];
+        float ti;
+        if (!slab(r.o, winv, r.tmin, far_, in.mn[0], in.mn[1], in.mn[2], in.mx[0], in.mx[1], in.mx[2], ti)) continue;
+        if ((r.mask & in.mask) == 0u) continue;
+        fl = merge_flags(r.flags, in.flags);
+        if (fl & F_SKIP_TRIANGLES) continue;
+        F3 bd;
+        object_ray(in.inv, r.o, r.d, o, bd, s);
+        stk.set_ray(o, bd);
+        inv = recip(bd);
+        near_ = r.tmin * s;
+        g = in.geo_begin;
+        gend = in.geo_end;
+      }
     }
   }
-  best.t = far_;  // far shrinks to each accepted hit
-  write_result(p, p.tri_ids, rid, best, cn, ct, ci);
 }
+
+// The register bound of a launch that asks for occupancy (TraceTune::waves):
+// 96 registers, 5 waves per SIMD.  At 6 or 8 waves the kernels spill inside
+// their loops (1080p frame 1.86 ms at 5 waves, 1.95 at 6; ambient-occlusion
+// sample, whose launches are the cooperative kernel's, 468 us at 5, 487 at 4,
+// 535 at 6; 1M rays in 100k triangles 336 us at 5, 352 at 6, 427 at 4).
+constexpr int kWavesBound = 5;
 
 // Live slots of the first and the second segment of a launch.
 __device__ __forceinline__ uint32_t live_first(const TraceParams &p) {
@@ -500,6 +760,10 @@ __device__ __forceinline__ void select_second(TraceParams &p) {
 constexpr uint32_t kCoopLanes = 8;
 constexpr uint32_t kCoopWideLanes = 16;
 constexpr uint32_t kCoopWideMax = 32768;
+// Inner steps go on while 1 / kCoopKeep of the wave's busy lanes want them
+// (2, 3, 6: 1.95, 1.97, 1.97 ms for the 1080p frame, 535, 538, 549 us for an
+// ambient-occlusion sample).
+constexpr uint32_t kCoopKeep = 2;
 
 template <int G>
 __device__ __forceinline__ float group_min(float v) {
@@ -518,94 +782,100 @@ __device__ __forceinline__ bool group_any(bool b) {
 constexpr uint32_t kCoopHit = 0x100u;
 
 template <int K, int S, int B, int LAYOUT, int G = (int)kCoopLanes>
-__device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_t rid, uint32_t *stk,
+__device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_t rid, uint32_t *lds,
                                                    uint32_t glane) {
   // the group's hit mask below is a 32-bit (1 << G) - 1
   static_assert(G == 8 || G == 16, "cooperative groups of 8 or 16 lanes");
-  uint32_t spill[S > K ? S - K : 1];
-  auto push = [&](uint32_t &sp, uint32_t v) {
-    if (sp < (uint32_t)K) stk[sp * B] = v;
-    else if (sp < (uint32_t)S) spill[sp - K] = v;
-    else {
-      atomicOr(p.status, 1u);  // unreachable when S covers the built depth
-      return;
-    }
-    sp++;
-  };
-  auto pop = [&](uint32_t &sp) -> uint32_t {
-    sp--;
-    return sp < (uint32_t)K ? stk[sp * B] : spill[sp - K];
-  };
+  volatile uint32_t spill[LaneStack<K, S, B>::kSpill];
+  LaneStack<K, S, B> stk{lds, spill, p.status, 0u};
 
   RayIn r = load_ray(p, rid);
   float far_ = r.tmax;  // group-uniform outside a batch's BLAS walks
   Best best;
   float best_t = 0.0f;  // this lane's own nearest accepted hit
   bool done = false;
-  uint32_t cand = kInvalid, cnt = 0, sp = 0;
+  uint32_t cand = kInvalid, cnt = 0;
 
-  // this lane's instance of the batch (already accepted by the TLAS walk)
+  // this lane's instance of the batch (already accepted by the TLAS walk);
+  // as in trace_wave the lanes of the wave do one kind of work at a time
   auto run_instance = [&](uint32_t i) {
     const InstRec &in = p.insts[i];
     const uint32_t fl = merge_flags(r.flags, in.flags);
-    F3 bo, bd;
     float s;
-    object_ray(in.inv, r.o, r.d, bo, bd, s);
-    const F3 binv = recip(bd);
+    {
+      F3 bo, bd;
+      object_ray(in.inv, r.o, r.d, bo, bd, s);
+      stk.set_ray(bo, bd);
+    }
     const float near_s = r.tmin * s;
-    bool ce, cb;
-    cull_triangle(fl, ce, cb);
-    for (uint32_t g = in.geo_begin; g < in.geo_end && !done; g++) {
-      const GeoRec &geo = p.geos[g];
-      if (!geometry_passes(fl, geo.flags)) continue;
-      const bool opq = geometry_opaque(fl, geo.flags);
-      float tg;
-      if (!slab(bo, binv, near_s, far_ * s, geo.mn[0], geo.mn[1], geo.mn[2], geo.mx[0], geo.mx[1], geo.mx[2], tg))
-        continue;
-      uint32_t bsp = sp;  // above the TLAS entries
-      uint32_t bref = LAYOUT ? geo.quad_root : geo.root_ref;
-      auto push_blas = [&](uint32_t v) { push(bsp, v); };
-      for (;;) {
-        if (!(bref & kLeafBit)) {
-          const float fs = far_ * s;
-          if constexpr (LAYOUT == 2) {
-            if (step_qquad(p.tri_qquads, bref, bo, binv, near_s, fs, push_blas)) continue;
-          } else if constexpr (LAYOUT == 1) {
-            if (step_quad(p.tri_quads, bref, bo, binv, near_s, fs, push_blas)) continue;
-          } else {
-            if (step_pair(p.tri_pairs, bref, bo, binv, near_s, fs, push_blas)) continue;
-          }
-        } else {
-          const uint32_t k0 = (bref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (bref & kLeafMaxCount);
-          for (uint32_t k = k0; k < k1; k++) {
-            const float4 *q = reinterpret_cast<const float4 *>(p.tris + k);
-            float4 a = q[0], b = q[1], c = q[2], d = q[3];
-            float t, u, v;
-            bool back;
-            if (tri_core(bo, bd, near_s, far_ * s, f3(a.x, a.y, a.z), f3(b.x, b.y, b.z), f3(c.x, c.y, c.z),
-                         f3(d.x, d.y, d.z), a.w, b.w, c.w, d.w, ce, cb, t, u, v, back)) {
-              uint32_t beh = opq ? RDRT_ANYHIT_ACCEPT : anyhit_behavior(p, false, p.tri_ids[k]);
-              if (beh & RDRT_ANYHIT_ACCEPT) {
-                far_ = t / s;
-                best_t = far_;
-                best.k = k;
-                best.geo = g;
-                best.inst = i;
-                best.u = u;
-                best.v = v;
-                best.back = back;
-                if (fl & F_END_SEARCH) beh |= RDRT_ANYHIT_END_SEARCH;
-              }
-              if (beh & RDRT_ANYHIT_END_SEARCH) {
-                done = true;
-                break;
-              }
+    uint32_t g = in.geo_begin, gend = in.geo_end, st = 0u, bref = kRefDone;
+    RayBox box = {};
+    // the first geometry from g on that the ray may hit
+    auto enter = [&]() {
+      F3 bo, bd;
+      stk.get_ray(bo, bd);
+      const F3 binv = recip(bd);
+      bref = kRefDone;
+      for (; g < gend; g++) {
+        const GeoRec &geo = p.geos[g];
+        float tg;
+        if (!geometry_passes(fl, geo.flags) || !slab(bo, binv, near_s, far_ * s, geo.mn[0], geo.mn[1], geo.mn[2],
+                                                     geo.mx[0], geo.mx[1], geo.mx[2], tg))
+          continue;
+        bool ce, cb;
+        cull_triangle(fl, ce, cb);
+        st = (geometry_opaque(fl, geo.flags) ? kStOpaque : 0u) | (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) |
+             ((fl & F_END_SEARCH) ? kStEnd : 0u);
+        box = ray_box(bo, binv);
+        stk.push(kRefExit);  // above the TLAS entries
+        bref = LAYOUT ? geo.quad_root : geo.root_ref;
+        break;
+      }
+    };
+    enter();
+    for (;;) {
+      const uint32_t a = wave_count(bref < kRefExit), b = wave_count((bref & kLeafBit) != 0u);
+      if (a + b == 0u) break;
+      if (a * kCoopKeep >= a + b) {
+        if (bref < kRefExit)
+          bref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, false, bref, box, near_s, far_ * s); });
+      } else if (bref & kLeafBit) {
+        const uint32_t k0 = (bref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (bref & kLeafMaxCount);
+        F3 bo, bd;
+        stk.get_ray(bo, bd);
+        bref = stk.pop();
+        for (uint32_t k = k0; k < k1; k++) {
+          const float4 *q = reinterpret_cast<const float4 *>(p.tris + k);
+          const float4 ta = q[0], tb = q[1], tc = q[2], td = q[3];
+          float t, u, v;
+          bool back;
+          if (tri_core(bo, bd, near_s, far_ * s, f3(ta.x, ta.y, ta.z), f3(tb.x, tb.y, tb.z), f3(tc.x, tc.y, tc.z),
+                       f3(td.x, td.y, td.z), ta.w, tb.w, tc.w, td.w, (st & kStCull) != 0u, (st & kStCullBack) != 0u, t,
+                       u, v, back)) {
+            uint32_t beh = (st & kStOpaque) ? RDRT_ANYHIT_ACCEPT : anyhit_behavior(p, false, p.tri_ids[k]);
+            if (beh & RDRT_ANYHIT_ACCEPT) {
+              far_ = t / s;
+              best_t = far_;
+              best.k = k;
+              best.geo = g;
+              best.inst = i;
+              best.u = u;
+              best.v = v;
+              best.back = back;
+              if (st & kStEnd) beh |= RDRT_ANYHIT_END_SEARCH;
+            }
+            if (beh & RDRT_ANYHIT_END_SEARCH) {
+              done = true;
+              bref = kRefDone;
+              break;
             }
           }
-          if (done) break;
         }
-        if (bsp == sp) break;
-        bref = pop(bsp);
+      }
+      if (bref == kRefExit) {
+        g++;
+        if (g < gend) enter();
+        else bref = kRefDone;
       }
     }
   };
@@ -625,16 +895,11 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
   if (root && slab(r.o, winv, r.tmin, far_, root->mn[0], root->mn[1], root->mn[2], root->mx[0], root->mx[1],
                    root->mx[2], tn)) {
     uint32_t ref = LAYOUT ? p.tlas_quad_roots[root - p.tlas_roots] : root->root_ref;
-    auto push_tlas = [&](uint32_t v) { push(sp, v); };
-    for (;;) {
+    stk.push(kRefDone);
+    RayBox box = ray_box(r.o, winv);
+    while (ref != kRefDone) {
       if (!(ref & kLeafBit)) {
-        if constexpr (LAYOUT == 2) {
-          if (step_qquad(p.tlas_qquads, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
-        } else if constexpr (LAYOUT == 1) {
-          if (step_quad(p.tlas_quads, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
-        } else {
-          if (step_pair(p.tlas_pairs, ref, r.o, winv, r.tmin, far_, push_tlas)) continue;
-        }
+        ref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, true, ref, box, r.tmin, far_); });
       } else {
         const uint32_t i0 = (ref & ~kLeafBit) >> kLeafCountBits, i1 = i0 + (ref & kLeafMaxCount);
         for (uint32_t i = i0; i < i1 && !done; i++) {
@@ -648,12 +913,12 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
           if (++cnt == (uint32_t)G) {
             flush();
             winv = recip(r.d);
+            box = ray_box(r.o, winv);
           }
         }
         if (done) break;
+        ref = stk.pop();
       }
-      if (sp == 0) break;
-      ref = pop(sp);
     }
     if (cnt) flush();
   }
@@ -687,9 +952,9 @@ __device__ __forceinline__ void trace_coop_group(TraceParams &p, uint32_t n0, ui
   trace_coop_one<K, S, B, LAYOUT, G>(p, rid, lds + threadIdx.x, threadIdx.x & ((uint32_t)G - 1u));
 }
 
-template <int K, int S, int B, int W, int LAYOUT>
-__global__ __launch_bounds__(B, W) void k_trace_coop(TraceParams p) {
-  __shared__ uint32_t lds[K * B];
+template <int K, int S, int B, int LAYOUT>
+__global__ __launch_bounds__(B, kWavesBound) void k_trace_coop(TraceParams p) {
+  __shared__ uint32_t lds[LaneStack<K, S, B>::kRows * B];
   const uint32_t n0 = live_first(p), n1 = live_second(p);
   if (n0 + n1 > p.coop_max) return;  // the one-ray-per-lane kernel traces launches this large
   // the group width is uniform over the launch (the live count is)
@@ -698,65 +963,70 @@ __global__ __launch_bounds__(B, W) void k_trace_coop(TraceParams p) {
 }
 
 // One ray per thread over a grid sized for both segments' slots; the live
-// counts may be smaller (device queue sizes).  The blocks of the second
-// segment follow those of the first, so a block's segment is uniform.
+// counts may be smaller (device queue sizes).
 template <int K, int S, int B, int W, bool CNT, int LAYOUT>
 __global__ __launch_bounds__(B, W) void k_trace_fast(TraceParams p) {
-  __shared__ uint32_t lds[K * B];
+  __shared__ uint32_t lds[LaneStack<K, S, B>::kRows * B];
   const uint32_t n0 = live_first(p), n1 = live_second(p);
   if (p.coop_max && n0 + n1 <= p.coop_max) return;  // the cooperative kernel traces it
-  const uint32_t b0 = (n0 + B - 1) / B;
-  const uint32_t used = b0 + (n1 + B - 1) / B;
+  const uint32_t total = n0 + n1, used = (total + B - 1) / B;
   if (blockIdx.x >= used) return;
-  uint32_t blk = xcd_block(blockIdx.x, used);
-  uint32_t n = n0;
-  if (blk >= b0) {
-    blk -= b0;
-    n = n1;
-    select_second(p);
-  }
-  const uint32_t slot = blk * B + threadIdx.x;
-  if (slot >= n) return;
-  const uint32_t rid = p.queue ? p.queue[slot] : slot;
-  if (rid >= p.n) return;  // a queue entry always names one of the n rays
-  trace_fast_one<K, S, B, CNT, LAYOUT>(p, rid, lds + threadIdx.x);
+  const uint32_t first = xcd_block(blockIdx.x, used) * B + (threadIdx.x & ~63u);
+  if (first >= total) return;  // whole waves
+  trace_wave<K, S, B, CNT, LAYOUT>(p, n0, __builtin_amdgcn_readfirstlane(first),
+                                   __builtin_amdgcn_readfirstlane(min(total, first + 64u)), lds + threadIdx.x,
+                                   [](uint32_t &, uint32_t &) { return false; });
 }
 
-// Persistent variant: a grid sized to the resident capacity; each wave
-// takes chunks of 64 consecutive queue slots from the device counter
-// p.work until the queue is exhausted, so uneven rays and scenes balance
-// across the chip.  Every wave exits once a fetch lands past the count.
-// The second segment's slots start at the first 64-aligned position after
-// the first segment's, so every chunk lies in one segment.
+// Persistent variant: a grid sized to the resident capacity whose waves pull
+// chunks of consecutive queue slots until the queue is exhausted, so uneven
+// rays and scenes balance across the chip.  The slots are divided among the
+// XCDs (blocks are dispatched to them round-robin), so that neighbouring rays
+// share an L2; a wave whose XCD's share is exhausted helps the next one.
+// Every share has a counter of its own: atomics on one address come out one
+// every ~18 ns, which on a single counter held a launch of 2M rays in chunks
+// of 64 at 0.7 ms whatever the rays took.  A wave's first chunk is the one of
+// its index, without an atomic.  Every wave exits once each share is drained.
 template <int K, int S, int B, int W, bool CNT, int LAYOUT>
 __global__ __launch_bounds__(B, W) void k_trace_persist(TraceParams p) {
-  __shared__ uint32_t lds[K * B];
+  __shared__ uint32_t lds[LaneStack<K, S, B>::kRows * B];
   const uint32_t n0 = live_first(p), n1 = live_second(p);
   if (p.coop_max && n0 + n1 <= p.coop_max) return;  // the cooperative kernel traces it
-  const uint32_t start1 = (n0 + 63u) & ~63u;
-  const uint32_t total = n1 ? start1 + n1 : n0;
-  const uint32_t lane = threadIdx.x & 63u;
-  for (;;) {
-    uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(p.work, 64u);
-    base = __builtin_amdgcn_readfirstlane(__shfl(base, 0, 64));  // wave-uniform: keeps q in scalar registers
-    if (base >= total) break;
-    TraceParams q = p;
-    uint32_t n = n0;
-    if (base >= start1) {
-      base -= start1;
-      n = n1;
-      select_second(q);
+  const uint32_t total = n0 + n1;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr uint32_t kWaves = B / 64u;
+  const uint32_t share = (total / kWorkGroups + 63u) & ~63u;  // slots of one XCD, in whole chunks
+  // chunks of 64, larger when a wave has very many to pull
+  const uint32_t chunk = total >= (1u << 22) ? 128u : 64u;
+  uint32_t tried = 0;      // shares found drained
+  bool own = true;         // the first chunk is not taken yet
+  trace_wave<K, S, B, CNT, LAYOUT>(p, n0, 0u, 0u, lds + threadIdx.x, [&](uint32_t &next, uint32_t &end) {
+    while (tried < kWorkGroups) {
+      const uint32_t g = (blockIdx.x + tried) % kWorkGroups;
+      const uint32_t first = g * share, stop = g + 1u == kWorkGroups ? total : min(total, first + share);
+      // the chunks of the group's own waves come first
+      const uint32_t waves = (gridDim.x - g + kWorkGroups - 1u) / kWorkGroups * kWaves;
+      uint32_t at;
+      if (own) {
+        own = false;
+        at = (blockIdx.x / kWorkGroups * kWaves + wave) * chunk;
+      } else {
+        uint32_t add = 0;
+        if (lane == 0) add = atomicAdd(p.work + g * kWorkStride, chunk);
+        at = waves * chunk + __builtin_amdgcn_readfirstlane(add);
+      }
+      if (first < stop && at < stop - first) {
+        next = first + at;
+        end = min(stop, next + chunk);
+        return true;
+      }
+      tried++;
     }
-    const uint32_t slot = base + lane;
-    if (slot < n) {
-      const uint32_t rid = q.queue ? q.queue[slot] : slot;
-      if (rid < q.n) trace_fast_one<K, S, B, CNT, LAYOUT>(q, rid, lds + threadIdx.x);
-    }
-  }
+    return false;
+  });
 }
 
-[[maybe_unused]] __global__ void k_zero_work(uint32_t *w) { *w = 0u; }
+[[maybe_unused]] __global__ void k_zero_work(uint32_t *w) { clear_work(w, threadIdx.x); }
 
 // One fast-traversal launch with block size B, total stack S and tuning t.
 // K = stack entries per lane in LDS, W = minimum waves per SIMD asked of the
@@ -773,12 +1043,12 @@ hipError_t launch_fast_kw(const TraceParams &p0, bool persist, uint32_t coop, hi
     // 8 lanes per ray, or 16 when at most kCoopWideMax rays are live
     const uint32_t threads = std::max(groups * kCoopLanes, std::min(groups, kCoopWideMax) * kCoopWideLanes);
     const uint32_t grid = (threads + B - 1) / B;
-    if (grid) hipLaunchKernelGGL((k_trace_coop<K, S, B, W, LAYOUT>), dim3(grid), dim3(B), 0, st, p);
+    if (grid) hipLaunchKernelGGL((k_trace_coop<K, S, B, LAYOUT>), dim3(grid), dim3(B), 0, st, p);
     if (live <= p.coop_max) return hipGetLastError();  // the cooperative kernel always qualifies
   }
   if (persist) {
     if (!p.work) return hipErrorInvalidValue;
-    if (!p.work_zeroed) hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(1), 0, st, p.work);
+    if (!p.work_zeroed) hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(64), 0, st, p.work);
     if (p.counters) {
       auto k = k_trace_persist<K, S, B, W, true, LAYOUT>;
       uint32_t g = std::min(resident_grid((const void *)k, B), grid_slots(p, B) / B);
@@ -801,13 +1071,9 @@ hipError_t launch_fast_s(const TraceParams &p, const TraceTune &t, hipStream_t s
   constexpr int K8 = S < 8 ? S : 8;
   constexpr int K16 = S < 16 ? S : 16;
   const bool persist = t.persist != 0;
-  if (t.waves >= 8) {
-    if (t.lds <= 8) return launch_fast_kw<K8, S, B, 8, LAYOUT>(p, persist, t.coop, st);
-    return launch_fast_kw<K16, S, B, 8, LAYOUT>(p, persist, t.coop, st);
-  }
-  if (t.waves >= 6) {
-    if (t.lds <= 8) return launch_fast_kw<K8, S, B, 6, LAYOUT>(p, persist, t.coop, st);
-    return launch_fast_kw<K16, S, B, 6, LAYOUT>(p, persist, t.coop, st);
+  if (t.waves) {
+    if (t.lds <= 8) return launch_fast_kw<K8, S, B, kWavesBound, LAYOUT>(p, persist, t.coop, st);
+    return launch_fast_kw<K16, S, B, kWavesBound, LAYOUT>(p, persist, t.coop, st);
   }
   if (t.lds <= 8) return launch_fast_kw<K8, S, B, 1, LAYOUT>(p, persist, t.coop, st);
   return launch_fast_kw<K16, S, B, 1, LAYOUT>(p, persist, t.coop, st);

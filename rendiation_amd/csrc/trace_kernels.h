@@ -9,6 +9,16 @@
 
 namespace rdrt {
 
+// Work counters of a persistent traversal launch: one per XCD, each on a line
+// of its own.
+constexpr uint32_t kWorkGroups = 8, kWorkStride = 32, kWorkWords = kWorkGroups * kWorkStride;
+#ifdef __HIP__
+// Clears the counters: thread i of one block, i < kWorkGroups at least.
+__device__ __forceinline__ void clear_work(uint32_t *work, uint32_t i) {
+  if (i < kWorkGroups) work[i * kWorkStride] = 0u;
+}
+#endif
+
 // Device view of a committed scene plus one launch's I/O.
 struct TraceParams {
   const rdrt_ray *rays;
@@ -25,7 +35,7 @@ struct TraceParams {
   const uint32_t *count;
   uint32_t slots;  // queue slots the grid covers (0 = n); ray ids stay < n
   uint2 *hitx;     // optional: (global geometry index, forest instance index) per hit
-  uint32_t *work;  // device work counter of the persistent kernel
+  uint32_t *work;  // device work counters of the persistent kernel (kWorkWords)
   // Optional second segment traced by the same launch (fast traversal
   // only): queue2[0 .. min(slots2, *count2)) with its own rays, hits, hit
   // extras and flags; ray ids index rays2 / hits2 and stay < n.  The
@@ -46,7 +56,7 @@ struct TraceParams {
   // (0 = their slots): when coop_max reaches it, only the cooperative kernel
   // is launched.
   uint32_t live_max;
-  // 1: the caller's previous kernel on the stream left *work at zero, so a
+  // 1: the caller's previous kernel on the stream cleared the counters, so a
   // persistent launch needs no clearing launch first
   uint32_t work_zeroed;
 
@@ -90,8 +100,9 @@ uint32_t stack_entries_for(uint32_t push_depth);
 struct TraceTune {
   uint32_t block = 256;  // threads per block: 64, 128 or 256
   uint32_t lds = 16;     // stack entries per lane kept in LDS: 8 or 16 (deeper ones in private memory)
-  uint32_t waves = 0;    // 8 / 6 = ask the register allocator for 8 / 6 waves per SIMD; 0 = its own choice
-  uint32_t persist = 0;  // 1 = resident-size grid whose waves pull 64-ray chunks from a counter
+  uint32_t waves = 0;    // 6 or 8 = bound the registers for occupancy (5 waves per SIMD, see kWavesBound);
+                         //     0 = the compiler's own choice
+  uint32_t persist = 0;  // 1 = resident-size grid whose waves pull chunks of rays from counters
   uint32_t cull = 0;     // 1 = a first pass finishes the rays that miss their scene's root box and
                          //     queues the others densely for the traversal
   uint32_t wide = 0;     // node layout: 0 = child pairs, 1 = child quads (four boxes per node),
