@@ -503,7 +503,7 @@ int32_t rdrt_pt_backward_geometry(rdrt_ctx *c, const float *adj, float *grad_pos
   L.g_nrm = grad_nrm;  // zeroed by the replay; stays zero without vertex normals
   L.nvertices = (uint32_t)(c->dev.vertices.count / 3);
   DetBufs db;
-  rc = reserve_det(s, 6 * (size_t)L.nvertices, db);
+  rc = reserve_det(s, 8 * (size_t)L.nvertices, db);
   if (rc) return rc;
   RDRT_HIP(s.grec.reserve(std::max<size_t>((size_t)L.max_bounces * L.npaths, 1) * 3 * sizeof(uint4)));
   L.grec = (uint4 *)s.grec.ptr;

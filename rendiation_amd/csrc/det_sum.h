@@ -15,7 +15,8 @@
 //
 // Protocol per accumulation (all on one stream):
 //   k_det_clear -> terms: det_note_max (pass 1) -> k_det_scale ->
-//   terms: det_add (pass 2) -> k_det_finish.
+//   terms: det_quant added to the entry, or special_of or-ed to its flags
+//   (pass 2) -> k_det_finish.
 #ifndef RDRT_DET_SUM_H
 #define RDRT_DET_SUM_H
 
@@ -46,10 +47,14 @@ __device__ __forceinline__ uint32_t abs_bits(float x) {
   return b < 0x7f800000u ? b : 0u;
 }
 
-// Wave-wide max of per-lane bits, then one atomic per wave.
+// Wave-wide max of per-lane bits, then one atomic for a wave that exceeds what
+// is noted already (a stale read only costs an atomic).  With an atomic per
+// wave the one address bound the launch: shading 8.4M replayed paths took 1.03
+// instead of 0.45 ms, the first pass over 1M recorded paths 59 instead of 21 us.
 __device__ __forceinline__ void det_note_max(Header *h, uint32_t bits) {
   for (int off = 32; off > 0; off >>= 1) bits = max(bits, (uint32_t)__shfl_xor((int)bits, off, 64));
-  if ((threadIdx.x & 63u) == 0 && bits) atomicMax(&h->maxbits, bits);
+  if ((threadIdx.x & 63u) == 0 && bits > __hip_atomic_load(&h->maxbits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(&h->maxbits, bits);
 }
 
 __device__ __forceinline__ uint32_t special_of(float x) {
@@ -57,18 +62,7 @@ __device__ __forceinline__ uint32_t special_of(float x) {
   return x > 0.0f ? kPosInf : kNegInf;
 }
 
-// One term into entry i (acc: int64 sums as u64, flags: non-finite marks).
-__device__ __forceinline__ void det_add(u64 *acc, uint32_t *flags, size_t i, float x, int32_t e) {
-  if (x == 0.0f) return;
-  if ((__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) {
-    atomicOr(flags + i, special_of(x));
-    return;
-  }
-  const long long q = __double2ll_rn((double)x * pow2(e));
-  atomicAdd(acc + i, (u64)q);
-}
-
-// The integer a term adds (callers that sum block-locally first).
+// The integer a finite term adds to its entry's sum.
 __device__ __forceinline__ long long det_quant(float x, int32_t e) { return __double2ll_rn((double)x * pow2(e)); }
 __device__ __forceinline__ bool det_finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
 
@@ -85,8 +79,9 @@ inline uint32_t ceil_log2(uint64_t n) {
 // the non-finite value the flags call for.
 hipError_t enqueue_clear(u64 *acc, uint32_t *flags, size_t n, Header *h, hipStream_t st);
 hipError_t enqueue_scale(Header *h, uint64_t max_terms_per_entry, hipStream_t st);
+// `stride`: distance of consecutive triples of entries (3: they are contiguous).
 hipError_t enqueue_finish(const u64 *acc, const uint32_t *flags, size_t n, const Header *h, float *out,
-                          hipStream_t st);
+                          hipStream_t st, uint32_t stride = 3);
 
 }  // namespace det
 }  // namespace rdrt

@@ -32,16 +32,18 @@ __global__ void k_det_scale(Header *h, uint32_t log2_terms) {
   h->e = 62 - (int32_t)log2_terms - ub;
 }
 
-__global__ void k_det_finish(const u64 *acc, const uint32_t *flags, size_t n, const Header *h, float *out) {
+__global__ void k_det_finish(const u64 *acc, const uint32_t *flags, size_t n, const Header *h, float *out,
+                             uint32_t stride3) {
   const double inv = pow2(-h->e);
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const uint32_t f = flags[i];
+    const size_t at = i / 3 * stride3 + i % 3;
+    const uint32_t f = flags[at];
     float v;
     if (f & kNaN || (f & kPosInf && f & kNegInf)) v = __uint_as_float(0x7fc00000u);
     else if (f & kPosInf) v = __uint_as_float(0x7f800000u);
     else if (f & kNegInf) v = __uint_as_float(0xff800000u);
-    else v = (float)((double)(long long)acc[i] * inv);
+    else v = (float)((double)(long long)acc[at] * inv);
     out[i] = v;
   }
 }
@@ -67,9 +69,9 @@ hipError_t enqueue_scale(Header *h, uint64_t max_terms_per_entry, hipStream_t st
 }
 
 hipError_t enqueue_finish(const u64 *acc, const uint32_t *flags, size_t n, const Header *h, float *out,
-                          hipStream_t st) {
+                          hipStream_t st, uint32_t stride) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_det_finish, dim3(grid_for(n)), dim3(256), 0, st, acc, flags, n, h, out);
+  hipLaunchKernelGGL(k_det_finish, dim3(grid_for(n)), dim3(256), 0, st, acc, flags, n, h, out, stride);
   return hipGetLastError();
 }
 

@@ -114,7 +114,7 @@ hipError_t enqueue_pt_backward(const PtLaunch &L, const float *adj, float *grad_
 // Replays the recorded frame L (same kernels, no shadow rays), records the
 // gradient terms of every bounce in L.grec and writes the gradient w.r.t.
 // vertex positions and normals to L.g_pos / L.g_nrm (g_nrm may be null).
-// Reproducible: db holds 6 * nvertices sums.
+// Reproducible: db holds 8 * nvertices sums (6 used, one line per vertex).
 hipError_t enqueue_pt_replay(const PtLaunch &L, const TraceParams &scene_tp, uint32_t push_depth,
                              const TraceTune &tune, const DetBufs &db, hipStream_t stream);
 // Packs device albedo / emission arrays (n * 3 each) into Material records.
