@@ -247,6 +247,11 @@ struct Kids {
 // move outwards, so a node test may pass a box that the exact test fails,
 // never the other way round.  |inv| is bounded (2^60), so that an axis-parallel
 // ray gets large finite distances and no NaN on that axis.
+//
+// The child-pair layout keeps the reference's arithmetic, (plane - o) * inv
+// (RayBox::nb is the origin there, fb unused): its two tests gain nothing from
+// the fused form, and on grids of axis-aligned edges the exact form decides
+// thousands of rays that pass within rounding of an edge.
 struct RayBox {
   F3 inv, nb, fb;
 };
@@ -257,8 +262,10 @@ __device__ __forceinline__ void ray_box_axis(float o, float inv, float &iv, floa
   nb = c - e;
   fb = c + e;
 }
+template <int LAYOUT>
 __device__ __forceinline__ RayBox ray_box(F3 o, F3 inv) {
   RayBox r;
+  if constexpr (LAYOUT == 0) return RayBox{inv, o, f3(0.0f, 0.0f, 0.0f)};
   ray_box_axis(o.x, inv.x, r.inv.x, r.nb.x, r.fb.x);
   ray_box_axis(o.y, inv.y, r.inv.y, r.nb.y, r.fb.y);
   ray_box_axis(o.z, inv.z, r.inv.z, r.nb.z, r.fb.z);
@@ -280,12 +287,9 @@ __device__ __forceinline__ bool box_hit(const RayBox &r, float tmin, float tmax,
 __device__ __forceinline__ Kids kids_pair(const PairNode *node, const RayBox &r, float tmin, float tmax) {
   const float4 *q = reinterpret_cast<const float4 *>(node);
   const float4 a = q[0], b = q[1], c = q[2], d = q[3];
-  const bool sx = negative(r.inv.x), sy = negative(r.inv.y), sz = negative(r.inv.z);
   float tl, tr;
-  const bool hl = box_hit(r, tmin, tmax, sx ? b.x : a.x, sy ? b.y : a.y, sz ? b.z : a.z, sx ? a.x : b.x,
-                          sy ? a.y : b.y, sz ? a.z : b.z, tl);
-  const bool hr = box_hit(r, tmin, tmax, sx ? d.x : c.x, sy ? d.y : c.y, sz ? d.z : c.z, sx ? c.x : d.x,
-                          sy ? c.y : d.y, sz ? c.z : d.z, tr);
+  const bool hl = slab(r.nb, r.inv, tmin, tmax, a.x, a.y, a.z, b.x, b.y, b.z, tl);
+  const bool hr = slab(r.nb, r.inv, tmin, tmax, c.x, c.y, c.z, d.x, d.y, d.z, tr);
   const uint32_t lref = __float_as_uint(a.w), rref = __float_as_uint(c.w);
   const bool rlast = hr && (!hl || tr < tl);  // the right child is the nearest hit
   Kids k;
@@ -491,8 +495,8 @@ constexpr uint32_t kRefExit = 0x7ffffff0u;  // the lane's BLAS is exhausted
 constexpr uint32_t kRefDone = 0x7ffffff1u;  // the lane's ray is finished (or it has none)
 // lane status bits
 constexpr uint32_t kStOpaque = 1u, kStCull = 2u, kStCullBack = 4u, kStEnd = 8u, kStSecond = 16u, kStBack = 32u,
-                   kStWorld = 64u;
-constexpr uint32_t kStMoreShift = 8;  // instances of the TLAS leaf still to visit
+                   kStWorld = 64u, kStGeometries = 128u;  // kStGeometries: geometries of the instance are left to visit
+constexpr uint32_t kStMoreShift = 8;                      // instances of the TLAS leaf still to visit
 
 __device__ __forceinline__ uint32_t wave_rank(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -512,6 +516,11 @@ constexpr uint32_t kRefill = 32;
 // 4.42, 4.15, 4.51, 4.50 ms for a batch of 16 scenes, measured on an earlier
 // build of these kernels).
 constexpr uint32_t kKeep = 3;
+// Leaves go before instances unless the lanes at instances outnumber those at
+// leaves by more than this: an instance step costs twice a leaf's, so it waits
+// for company (1, 2, 4: 500, 482, 474 us for a small-mesh material step, 15.96,
+// 15.86, 15.72 ms for a height-field step, 2.32, 2.26, 2.28 ms for a batch).
+constexpr uint32_t kLeavesFirst = 3;
 
 template <int K, int S, int B, bool CNT, int LAYOUT, class More>
 __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, uint32_t next, uint32_t end,
@@ -574,7 +583,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
         if (rid < p.n) {  // a queue entry always names one of the n rays
           const RayIn r = ray_of();
           const F3 winv = recip(r.d);
-          box = ray_box(r.o, winv);
+          box = ray_box<LAYOUT>(r.o, winv);
           near_ = r.tmin;
           far_ = r.tmax;
           s = 1.0f;
@@ -609,7 +618,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
       continue;
     }
     const bool leaf = (ref & kLeafBit) != 0u, world = (st & kStWorld) != 0u;
-    if (wave_count(leaf && !world) >= wave_count(ref == kRefExit || (leaf && world))) {
+    if (kLeavesFirst * wave_count(leaf && !world) >= wave_count(ref == kRefExit || (leaf && world))) {
       if (leaf && !world) {
         const uint32_t k0 = (ref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (ref & kLeafMaxCount);
         F3 o, bd;
@@ -656,11 +665,12 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
         g = gend = fl = 0u;
       } else {
         left = st >> kStMoreShift;
-        const InstRec &in = p.insts[inst];
-        g = geo + 1u;
-        gend = in.geo_end;
-        fl = merge_flags(r.flags, in.flags);
-        if (g < gend) {
+        g = gend = fl = 0u;
+        if (st & kStGeometries) {
+          const InstRec &in = p.insts[inst];
+          g = geo + 1u;
+          gend = in.geo_end;
+          fl = merge_flags(r.flags, in.flags);
           F3 bd;
           stk.get_ray(o, bd);
           inv = recip(bd);
@@ -676,9 +686,9 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
             cull_triangle(fl, ce, cb);
             st = (st & (kStSecond | kStBack)) | (geometry_opaque(fl, gr.flags) ? kStOpaque : 0u) |
                  (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) | ((fl & F_END_SEARCH) ? kStEnd : 0u) |
-                 (left << kStMoreShift);
+                 (g + 1u < gend ? kStGeometries : 0u) | (left << kStMoreShift);
             geo = g;
-            box = ray_box(o, inv);
+            box = ray_box<LAYOUT>(o, inv);
             stk.push(kRefExit);  // the end mark of the BLAS, above the TLAS entries
             ref = LAYOUT ? gr.quad_root : gr.root_ref;
             break;
@@ -687,7 +697,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
           continue;
         }
         if (left == 0u) {
-          box = ray_box(r.o, winv);
+          box = ray_box<LAYOUT>(r.o, winv);
           near_ = r.tmin;
           s = 1.0f;
           st |= kStWorld;
@@ -826,7 +836,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
         cull_triangle(fl, ce, cb);
         st = (geometry_opaque(fl, geo.flags) ? kStOpaque : 0u) | (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) |
              ((fl & F_END_SEARCH) ? kStEnd : 0u);
-        box = ray_box(bo, binv);
+        box = ray_box<LAYOUT>(bo, binv);
         stk.push(kRefExit);  // above the TLAS entries
         bref = LAYOUT ? geo.quad_root : geo.root_ref;
         break;
@@ -896,7 +906,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
                    root->mx[2], tn)) {
     uint32_t ref = LAYOUT ? p.tlas_quad_roots[root - p.tlas_roots] : root->root_ref;
     stk.push(kRefDone);
-    RayBox box = ray_box(r.o, winv);
+    RayBox box = ray_box<LAYOUT>(r.o, winv);
     while (ref != kRefDone) {
       if (!(ref & kLeafBit)) {
         ref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, true, ref, box, r.tmin, far_); });
@@ -913,7 +923,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
           if (++cnt == (uint32_t)G) {
             flush();
             winv = recip(r.d);
-            box = ray_box(r.o, winv);
+            box = ray_box<LAYOUT>(r.o, winv);
           }
         }
         if (done) break;
@@ -962,19 +972,34 @@ __global__ __launch_bounds__(B, kWavesBound) void k_trace_coop(TraceParams p) {
   else trace_coop_group<K, S, B, LAYOUT, (int)kCoopLanes>(p, n0, n1, lds);
 }
 
-// One ray per thread over a grid sized for both segments' slots; the live
-// counts may be smaller (device queue sizes).
+// Rays that a wave starts with.  A launch that leaves SIMDs idle lasts as long
+// as its slowest wave, and a wave takes the steps of all its rays, so few rays
+// go to each, until there are two waves per SIMD (4096 rays in 2000 triangles:
+// 59.6 us in 64 waves of 64, 47.0 in 512 of 8; 21k paths in 64 meshes: 477 and
+// 419 us; 1024 or 4096 waves are within 4 % of 2048).
+constexpr uint32_t kSpreadWaves = 2048, kFewestRays = 8;
+__host__ __device__ inline uint32_t rays_per_wave(uint32_t total, uint32_t waves) {
+  uint32_t r = kFewestRays;
+  const uint32_t w = waves < kSpreadWaves ? waves : kSpreadWaves;
+  while (r < 64u && (total + r - 1u) / r > w) r *= 2u;
+  return r;
+}
+
+// One ray per thread, or fewer rays than lanes in a small launch, over a grid
+// sized for both segments' slots; the live counts may be smaller (device queue
+// sizes).
 template <int K, int S, int B, int W, bool CNT, int LAYOUT>
 __global__ __launch_bounds__(B, W) void k_trace_fast(TraceParams p) {
   __shared__ uint32_t lds[LaneStack<K, S, B>::kRows * B];
   const uint32_t n0 = live_first(p), n1 = live_second(p);
   if (p.coop_max && n0 + n1 <= p.coop_max) return;  // the cooperative kernel traces it
-  const uint32_t total = n0 + n1, used = (total + B - 1) / B;
+  const uint32_t total = n0 + n1, per = rays_per_wave(total, gridDim.x * (B / 64u)), block = per * (B / 64u);
+  const uint32_t used = (total + block - 1u) / block;
   if (blockIdx.x >= used) return;
-  const uint32_t first = xcd_block(blockIdx.x, used) * B + (threadIdx.x & ~63u);
+  const uint32_t first = xcd_block(blockIdx.x, used) * block + (threadIdx.x >> 6) * per;
   if (first >= total) return;  // whole waves
   trace_wave<K, S, B, CNT, LAYOUT>(p, n0, __builtin_amdgcn_readfirstlane(first),
-                                   __builtin_amdgcn_readfirstlane(min(total, first + 64u)), lds + threadIdx.x,
+                                   __builtin_amdgcn_readfirstlane(min(total, first + per)), lds + threadIdx.x,
                                    [](uint32_t &, uint32_t &) { return false; });
 }
 
@@ -996,8 +1021,9 @@ __global__ __launch_bounds__(B, W) void k_trace_persist(TraceParams p) {
   const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr uint32_t kWaves = B / 64u;
   const uint32_t share = (total / kWorkGroups + 63u) & ~63u;  // slots of one XCD, in whole chunks
-  // chunks of 64, larger when a wave has very many to pull
-  const uint32_t chunk = total >= (1u << 22) ? 128u : 64u;
+  // chunks of 64, larger when a wave has very many to pull, smaller when the
+  // first ones already leave waves without rays
+  const uint32_t chunk = total >= (1u << 22) ? 128u : rays_per_wave(total, gridDim.x * kWaves);
   uint32_t tried = 0;      // shares found drained
   bool own = true;         // the first chunk is not taken yet
   trace_wave<K, S, B, CNT, LAYOUT>(p, n0, 0u, 0u, lds + threadIdx.x, [&](uint32_t &next, uint32_t &end) {
@@ -1026,6 +1052,13 @@ __global__ __launch_bounds__(B, W) void k_trace_persist(TraceParams p) {
   });
 }
 
+// Blocks of a launch: a lane for every slot, or a wave for every kFewestRays
+// slots of a launch too small for kSpreadWaves waves of 64.
+inline uint32_t spread_grid(const TraceParams &p, uint32_t block) {
+  const uint32_t blocks = grid_slots(p, block) / block, most = (kSpreadWaves * 64u + block - 1u) / block;
+  return blocks >= most ? blocks : std::min(most, blocks * (64u / kFewestRays));
+}
+
 [[maybe_unused]] __global__ void k_zero_work(uint32_t *w) { clear_work(w, threadIdx.x); }
 
 // One fast-traversal launch with block size B, total stack S and tuning t.
@@ -1051,16 +1084,16 @@ hipError_t launch_fast_kw(const TraceParams &p0, bool persist, uint32_t coop, hi
     if (!p.work_zeroed) hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(64), 0, st, p.work);
     if (p.counters) {
       auto k = k_trace_persist<K, S, B, W, true, LAYOUT>;
-      uint32_t g = std::min(resident_grid((const void *)k, B), grid_slots(p, B) / B);
+      uint32_t g = std::min(resident_grid((const void *)k, B), spread_grid(p, B));
       hipLaunchKernelGGL(k, dim3(g), dim3(B), 0, st, p);
     } else {
       auto k = k_trace_persist<K, S, B, W, false, LAYOUT>;
-      uint32_t g = std::min(resident_grid((const void *)k, B), grid_slots(p, B) / B);
+      uint32_t g = std::min(resident_grid((const void *)k, B), spread_grid(p, B));
       hipLaunchKernelGGL(k, dim3(g), dim3(B), 0, st, p);
     }
     return hipGetLastError();
   }
-  dim3 grid(grid_slots(p, B) / B);
+  dim3 grid(spread_grid(p, B));
   if (p.counters) hipLaunchKernelGGL((k_trace_fast<K, S, B, W, true, LAYOUT>), grid, dim3(B), 0, st, p);
   else hipLaunchKernelGGL((k_trace_fast<K, S, B, W, false, LAYOUT>), grid, dim3(B), 0, st, p);
   return hipGetLastError();

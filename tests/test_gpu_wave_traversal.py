@@ -70,9 +70,9 @@ def test_ray_counts(device, n):
 
 
 def _ladder(count):
-    """Triangles across the x axis at x = 2^-i, sized by x: the trees are chains, whose quads need stacks of 16, 24
-    and 48 entries for 12, 24 and 40 triangles."""
-    x = np.float32(2.0) ** -np.arange(count, dtype=np.float32)
+    """Triangles across the x axis at x = 2^(10 - i), sized by x: the trees are chains, whose quads need stacks of 16,
+    24 and 48 entries for 12, 24 and 40 triangles.  (The products of four edge lengths stay normal numbers.)"""
+    x = np.float32(2.0) ** (10 - np.arange(count, dtype=np.float32))
     tri = np.zeros((count, 3, 3), dtype=np.float32)
     tri[:, :, 0] = x[:, None]
     tri[:, :, 1:] = np.array([[-1.0, -1.0], [1.0, -1.0], [0.0, 1.2]], dtype=np.float32) * x[:, None, None]
@@ -85,12 +85,12 @@ def test_deep_stacks(device, count, entries):
     assert s.scene_info().quad_stack_entries == entries
     rng = np.random.default_rng(count)
     n = 4096
-    size = np.float32(2.0) ** -rng.uniform(0.0, count, n)
+    size = np.float32(2.0) ** (10 - rng.uniform(0.0, count, n))
     rays = np.zeros((n, 8), dtype=np.float32)
-    rays[:, 0] = np.where(rng.random(n) < 0.7, -1.0, 2.0)  # towards the small end: the deepest child is the nearest
+    rays[:, 0] = np.where(rng.random(n) < 0.7, -1.0, 2000.0)  # towards the small end: the deepest child is the nearest
     rays[:, 1:3] = rng.uniform(-1.2, 1.2, (n, 2)) * size[:, None]
     rays[:, 4] = np.where(rays[:, 0] < 0, 1.0, -1.0)
-    rays[:, 5:7] = rng.uniform(-0.2, 0.2, (n, 2)) * size[:, None]
+    rays[:, 5:7] = rng.uniform(-1e-4, 1e-4, (n, 2)) * size[:, None]
     rays[:, 3], rays[:, 7] = 1e-6, np.inf
     want = _check(s, rays, "ladder")
     assert len(np.unique(want[:, 0])) > count // 2
