@@ -10,6 +10,7 @@
 
 #include <chrono>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -74,6 +75,7 @@ void release_refit(rdrt_ctx *c) {
   release(c->refit_pairs);
   release(c->refit_quads);
   c->refit_boxes.free();
+  c->refit_staging.free();
   c->refit_ready = false;
 }
 
@@ -158,14 +160,48 @@ uint32_t push_depth(const rdrt_ctx *c, const TraceTune &t) {
 
 namespace {
 
-// Replaces a device array with a new host array, keeping the byte count.
-template <class T>
-hipError_t reupload(DevArray<T> &a, const std::vector<T> &h, uint64_t &bytes) {
-  const uint64_t old = (uint64_t)(a.count ? a.count : 1) * sizeof(T);
-  if (a.ptr) bytes -= std::min(bytes, old);
-  release(a);
-  return upload(a, h, bytes);
-}
+// Replaces the contents of device arrays on a stream: in place where the size
+// is the same (a refit keeps every count unless the TLAS trees change shape),
+// from pinned staging so that the copies need not wait for each other.
+// finish() waits for them; nothing may reuse the staging before.
+class Reupload {
+ public:
+  Reupload(Pinned &staging, hipStream_t st, uint64_t &bytes) : p_(staging), st_(st), bytes_(bytes) {}
+  template <class T>
+  void add(DevArray<T> &a, const std::vector<T> &h) {
+    total_ += (h.size() * sizeof(T) + 15) & ~(size_t)15;
+    jobs_.push_back([this, &a, &h]() -> hipError_t {
+      const size_t n = h.size() * sizeof(T);
+      if (!a.ptr || a.count != h.size()) {
+        const uint64_t old = (uint64_t)(a.count ? a.count : 1) * sizeof(T);
+        if (a.ptr) bytes_ -= std::min(bytes_, old);
+        release(a);
+        return upload(a, h, bytes_);
+      }
+      if (n == 0) return hipSuccess;
+      char *src = (char *)p_.ptr + at_;
+      at_ += (n + 15) & ~(size_t)15;
+      std::memcpy(src, h.data(), n);
+      return hipMemcpyAsync(a.ptr, src, n, hipMemcpyHostToDevice, st_);
+    });
+  }
+  hipError_t finish() {
+    hipError_t e = p_.reserve(total_);
+    for (auto &job : jobs_) {
+      if (e != hipSuccess) break;
+      e = job();
+    }
+    const hipError_t w = hipStreamSynchronize(st_);
+    return e != hipSuccess ? e : w;
+  }
+
+ private:
+  Pinned &p_;
+  hipStream_t st_;
+  uint64_t &bytes_;
+  size_t total_ = 0, at_ = 0;
+  std::vector<std::function<hipError_t()>> jobs_;
+};
 
 // Captured frames and batched calls hold the scene's device pointers.
 void drop_captures(rdrt_ctx *c) {
@@ -530,6 +566,7 @@ int32_t rdrt_refit(rdrt_ctx *c, const float *positions, const float *normals) {
   a.pairs = d.tri_pairs.ptr;
   a.quads = d.tri_quads.ptr;
   a.qquads = d.tri_qquads.ptr;
+  a.nquads = (uint32_t)d.tri_quads.count;
   a.geos = d.geos.ptr;
   a.ngeos = (uint32_t)d.geos.count;
   a.forest_nodes = c->refit_forest.ptr;
@@ -555,16 +592,18 @@ int32_t rdrt_refit(rdrt_ctx *c, const float *positions, const float *normals) {
   rc = build_tlas_layer(c->src, b, err);
   if (rc != RDRT_OK) return fail(rc, err);
   drop_captures(c);
-  RDRT_HIP(reupload(d.insts, b.insts, d.bytes));
-  RDRT_HIP(reupload(d.inst_fwd, b.inst_fwd, d.bytes));
-  RDRT_HIP(reupload(d.tlas_forest, b.tlas_forest, d.bytes));
-  RDRT_HIP(reupload(d.tlas_pairs, b.tlas_pairs, d.bytes));
-  RDRT_HIP(reupload(d.tlas_quads, b.tlas_quads, d.bytes));
-  RDRT_HIP(reupload(d.tlas_qquads, b.tlas_qquads, d.bytes));
-  RDRT_HIP(reupload(d.tlas_roots, b.tlas_roots, d.bytes));
-  RDRT_HIP(reupload(d.tlas_quad_roots, b.tlas_quad_roots, d.bytes));
-  RDRT_HIP(reupload(d.inst_lookup, b.inst_lookup, d.bytes));
-  RDRT_HIP(reupload(d.tlas_inst_first, b.tlas_inst_first, d.bytes));
+  Reupload up(c->refit_staging, st, d.bytes);
+  up.add(d.insts, b.insts);
+  up.add(d.inst_fwd, b.inst_fwd);
+  up.add(d.tlas_forest, b.tlas_forest);
+  up.add(d.tlas_pairs, b.tlas_pairs);
+  up.add(d.tlas_quads, b.tlas_quads);
+  up.add(d.tlas_qquads, b.tlas_qquads);
+  up.add(d.tlas_roots, b.tlas_roots);
+  up.add(d.tlas_quad_roots, b.tlas_quad_roots);
+  up.add(d.inst_lookup, b.inst_lookup);
+  up.add(d.tlas_inst_first, b.tlas_inst_first);
+  RDRT_HIP(up.finish());
   return RDRT_OK;
 }
 

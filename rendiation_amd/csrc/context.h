@@ -67,6 +67,25 @@ struct Scratch {
   }
 };
 
+// Grow-only pinned host buffer.
+struct Pinned {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+  hipError_t reserve(size_t n) {
+    if (n <= bytes) return hipSuccess;
+    free();
+    const hipError_t e = hipHostMalloc(&ptr, n, hipHostMallocDefault);
+    if (e == hipSuccess) bytes = n;
+    else ptr = nullptr;
+    return e;
+  }
+  void free() {
+    if (ptr) (void)hipHostFree(ptr);
+    ptr = nullptr;
+    bytes = 0;
+  }
+};
+
 struct DeviceScene {
   DevArray<PairNode> tri_pairs, tlas_pairs;
   DevArray<QuadNode> tri_quads, tlas_quads;
@@ -162,6 +181,7 @@ struct rdrt_ctx {
   rdrt::DevArray<uint32_t> refit_forest, refit_pairs, refit_quads;
   std::vector<uint32_t> refit_forest_off, refit_pairs_off, refit_quads_off;
   rdrt::Scratch refit_boxes;
+  rdrt::Pinned refit_staging;  // the TLAS layer on its way to the device
   rdrt::AoState *ao = nullptr;  // created by the first rdrt_ao_render
 };
 

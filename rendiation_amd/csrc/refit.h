@@ -21,6 +21,7 @@ struct RefitArgs {
   PairNode *pairs;
   QuadNode *quads;
   QuadNodeQ *qquads;
+  uint32_t nquads;
   GeoRec *geos;
   uint32_t ngeos;
   // node indices per layout, deepest level first, and level boundaries
@@ -29,8 +30,8 @@ struct RefitArgs {
 };
 
 // Enqueues the whole BLAS refit on `stream`: triangle records and boxes, then
-// the reference forest, the child pairs and the child quads (with their
-// quantized twins) level by level, then the geometry boxes.
+// the reference forest, the child pairs and the child quads level by level,
+// then the quads' quantized twins and the geometry boxes.
 hipError_t enqueue_refit(const RefitArgs &a, const uint32_t *forest_off, uint32_t forest_levels,
                          const uint32_t *pair_off, uint32_t pair_levels, const uint32_t *quad_off,
                          uint32_t quad_levels, hipStream_t stream);
