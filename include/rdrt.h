@@ -734,7 +734,7 @@ int32_t rdrt_compact(rdrt_ctx *ctx, const uint32_t *mask_dev, uint32_t n, uint32
  * it is for callers that cannot allocate (code under HIP graph capture,
  * tight serving loops).  Same outputs as rdrt_compact, for n up to
  * RDRT_COMPACT_STATIC_MAX (larger n returns RDRT_ERR_CAPACITY).  Its scratch
- * is a fixed device array of the library (about 8.5 MB, held by each device
+ * is a fixed device array of the library (about 270 KB, held by each device
  * the library runs on until the process ends); every call on one device
  * shares it, so calls that overlap on one device (other streams, other
  * contexts, other threads) race and must be ordered by the caller.  Enqueued

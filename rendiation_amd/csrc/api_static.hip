@@ -1,8 +1,8 @@
 // api_static.hip -- rdrt_compact_static: the stable stream compaction of
 // rdrt_compact with no device allocation, for callers that cannot allocate
 // (code under HIP graph capture, tight serving loops).  Its scratch (the
-// block-local runs, block counts and offsets of the three-pass compaction)
-// is one file-scope device array of fixed size, sized for
+// ballot bits, counts and offsets of the compaction's tiles) is one
+// file-scope device array of fixed size, sized for
 // RDRT_COMPACT_STATIC_MAX elements.  Each device the library runs on holds
 // its own copy until the process ends; every call on one device shares it,
 // so calls that overlap on one device race.  Nothing in it needs clearing:
@@ -20,9 +20,7 @@ using namespace rdrt;
 namespace {
 
 constexpr uint32_t kMaxN = RDRT_COMPACT_STATIC_MAX;
-constexpr size_t kBlocks = ((size_t)kMaxN + kPtBlock - 1) / kPtBlock;
-// block-local runs (kBlocks * kPtBlock) + block counts + block offsets + 1
-constexpr size_t kWords = kBlocks * kPtBlock + 2 * kBlocks + 1;
+constexpr size_t kWords = compact_scratch_words(kMaxN);
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;

@@ -127,10 +127,14 @@ uint32_t l2_adjoint_parts(uint32_t n);
 hipError_t enqueue_l2_adjoint(const float *a, const float *b, uint32_t n, float *adj, double *loss, double *part,
                               hipStream_t stream);
 
-// Stable stream compaction of indices whose mask is non-zero (block-local
-// runs, a scan of the block counts, a scatter); out_count receives the kept
-// count.  `scratch` holds compact_scratch_words(n) u32.
-size_t compact_scratch_words(uint32_t n);
+// Stable stream compaction of indices whose mask is non-zero; out_count
+// receives the kept count.  `scratch` holds compact_scratch_words(n) u32,
+// 8-byte aligned: per tile its ballot bits, its count and its offset.  The mask
+// is read before anything is written, so out_idx may be the mask.
+constexpr uint32_t kCompactTile = 4096;
+constexpr size_t compact_scratch_words(uint32_t n) {
+  return (((size_t)n + kCompactTile - 1) / kCompactTile) * (kCompactTile / 32u + 2u) + 1;
+}
 hipError_t enqueue_compact(const uint32_t *mask, uint32_t n, uint32_t *out_idx, uint32_t *out_count,
                            uint32_t *scratch, hipStream_t stream);
 

@@ -204,7 +204,6 @@ __global__ __launch_bounds__(kPtBlock) void k_pt_finalize(PtLaunch P) {
   store3(P.out + 3 * (size_t)image_pixel(P, slot), s * inv);
 }
 
-// standalone stable compaction (same machinery as the shade kernel)
 __global__ void k_fill_u64(u64 *p, uint32_t n) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
 }
@@ -241,12 +240,98 @@ __global__ __launch_bounds__(kPtBlock) void k_sum_visits(const uint32_t *queue, 
   if (threadIdx.x == 0 && m) atomicMax(max_visits, m);
 }
 
-__global__ __launch_bounds__(kPtBlock) void k_compact(const uint32_t *mask, uint32_t n, uint32_t *tmp,
-                                                      uint32_t *cnt) {
-  const uint32_t bid = blockIdx.x;
-  const uint32_t i = bid * kPtBlock + threadIdx.x;
-  const bool keep = i < n && mask[i] != 0u;
-  block_compact2<kPtBlock>(keep, false, i, bid, tmp, nullptr, cnt, nullptr);
+// Standalone stable compaction of a mask, in tiles of kCompactTile elements: a
+// wave takes 16 rows of 64.  The first launch turns each row into a word of
+// ballot bits and counts the tile, so the mask is read once and the second
+// launch, which writes the indices in order, reads n / 8 bytes instead of it.
+// Bound by the launches at small n (n <= one tile: one launch) and by memory
+// at large n: 4.19M flags of 30 %, 22 MB in and out, 31 us with block-local
+// runs, a scan of 16k block counts and a copy; 14 us now.
+constexpr uint32_t kCompactRows = 16;
+static_assert(kCompactTile == kPtBlock * kCompactRows, "a row per wave and step");
+
+// Ballot of row k of the wave's tile part in lane k (k < kCompactRows).
+__device__ __forceinline__ u64 compact_rows(const uint32_t *mask, uint32_t n, size_t base) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t m[kCompactRows];
+  if (base + kCompactRows * 64u <= n) {  // whole rows: all loads in flight
+    const uint32_t *p = mask + base + lane;
+#pragma unroll
+    for (uint32_t k = 0; k < kCompactRows; k++) m[k] = p[k * 64u];
+  } else {
+#pragma unroll
+    for (uint32_t k = 0; k < kCompactRows; k++) {
+      const size_t i = base + k * 64u + lane;
+      m[k] = i < n ? mask[i] : 0u;
+    }
+  }
+  u64 mine = 0ull;
+#pragma unroll
+  for (uint32_t k = 0; k < kCompactRows; k++) {
+    const u64 b = __ballot(m[k] != 0u);
+    if (lane == k) mine = b;
+  }
+  return mine;
+}
+
+__global__ __launch_bounds__(kPtBlock) void k_compact_count(const uint32_t *mask, uint32_t n, u64 *bits,
+                                                            uint32_t *cnt) {
+  __shared__ uint32_t s_total;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const size_t row = (size_t)blockIdx.x * (kCompactTile / 64u) + wave * kCompactRows;
+  if (threadIdx.x == 0) s_total = 0u;
+  __syncthreads();
+  const u64 b = compact_rows(mask, n, row * 64u);
+  if (lane < kCompactRows) {
+    bits[row + lane] = b;
+    atomicAdd(&s_total, (uint32_t)__popcll(b));
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) cnt[blockIdx.x] = s_total;
+}
+
+// Writes the tile's indices from its offset on: off[tile], or the sum of the
+// counts before it, or 0 of a single tile (bits null: read from the mask).
+__global__ __launch_bounds__(kPtBlock) void k_compact_write(const uint32_t *mask, uint32_t n, const u64 *bits,
+                                                            const uint32_t *cnt, const uint32_t *off, uint32_t *out,
+                                                            uint32_t *total) {
+  __shared__ uint32_t s_before, s_wave[kPtBlock / 64];
+  const uint32_t tile = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const size_t row = (size_t)tile * (kCompactTile / 64u) + wave * kCompactRows;
+  if (threadIdx.x == 0) s_before = off ? off[tile] : 0u;
+  u64 b = 0ull;
+  if (!bits) b = compact_rows(mask, n, row * 64u);
+  else if (lane < kCompactRows) b = bits[row + lane];
+  __syncthreads();
+  if (bits && !off) {
+    uint32_t sum = 0;
+    for (uint32_t t = threadIdx.x; t < tile; t += kPtBlock) sum += cnt[t];
+    for (int o = 32; o > 0; o >>= 1) sum += (uint32_t)__shfl_xor((int)sum, o, 64);
+    if (lane == 0 && sum) atomicAdd(&s_before, sum);
+  }
+  // exclusive prefix of the wave's rows, then of the block's waves
+  const uint32_t own = (uint32_t)__popcll(b);
+  uint32_t incl = own;
+  for (int o = 1; o < (int)kCompactRows; o <<= 1) {
+    const uint32_t x = (uint32_t)__shfl_up((int)incl, o, 64);
+    if (lane >= (uint32_t)o) incl += x;
+  }
+  if (lane == kCompactRows - 1u) s_wave[wave] = incl;
+  __syncthreads();
+  uint32_t base = s_before;
+  for (uint32_t w = 0; w < wave; w++) base += s_wave[w];
+  const uint32_t excl = incl - own;
+#pragma unroll
+  for (uint32_t k = 0; k < kCompactRows; k++) {
+    const u64 r = __shfl(b, (int)k, 64);
+    const uint32_t at = base + (uint32_t)__shfl((int)excl, (int)k, 64);
+    if ((r >> lane) & 1ull) out[at + compact::lane_rank(r)] = (uint32_t)((row + k) * 64u + lane);
+  }
+  if (tile + 1u == gridDim.x && threadIdx.x == 0) {
+    uint32_t t = s_before;
+    for (uint32_t w = 0; w < kPtBlock / 64; w++) t += s_wave[w];
+    *total = t;
+  }
 }
 
 // ---- adjoint ----
@@ -612,26 +697,31 @@ hipError_t enqueue_l2_adjoint(const float *a, const float *b, uint32_t n, float 
   return hipGetLastError();
 }
 
-size_t compact_scratch_words(uint32_t n) {
-  const size_t nb = ((size_t)n + kPtBlock - 1) / kPtBlock;
-  return nb * kPtBlock + 2 * nb + 1;
-}
-
 hipError_t enqueue_compact(const uint32_t *mask, uint32_t n, uint32_t *out_idx, uint32_t *out_count,
                            uint32_t *scratch, hipStream_t st) {
-  const uint32_t nb = (n + kPtBlock - 1) / kPtBlock;
-  if (nb == 0) {
+  const uint32_t nt = (uint32_t)(((size_t)n + kCompactTile - 1) / kCompactTile);
+  if (nt == 0) {
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, st, out_count);
     return hipGetLastError();
   }
-  uint32_t *tmp = scratch, *cnt = scratch + (size_t)nb * kPtBlock, *off = cnt + nb;
-  hipLaunchKernelGGL(k_compact, dim3(nb), dim3(kPtBlock), 0, st, mask, n, tmp, cnt);
-  hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanThreads), 0, st, (const uint32_t *)nullptr, n, kPtBlock, cnt,
-                     (const uint32_t *)nullptr, off, (uint32_t *)nullptr, out_count, (uint32_t *)nullptr);
-  hipLaunchKernelGGL((k_scatter2<kPtBlock>), dim3(nb), dim3(kPtBlock), 0, st, (const uint32_t *)nullptr, n,
-                     (const uint32_t *)tmp, (const uint32_t *)nullptr, (const uint32_t *)cnt,
-                     (const uint32_t *)nullptr, (const uint32_t *)off, (const uint32_t *)nullptr, out_idx,
-                     (uint32_t *)nullptr, n);
+  u64 *bits = (u64 *)scratch;
+  uint32_t *cnt = scratch + (size_t)nt * (kCompactTile / 32u), *off = cnt + nt;
+  if (nt == 1) {
+    hipLaunchKernelGGL(k_compact_write, dim3(1), dim3(kPtBlock), 0, st, mask, n, (const u64 *)nullptr,
+                       (const uint32_t *)nullptr, (const uint32_t *)nullptr, out_idx, out_count);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_compact_count, dim3(nt), dim3(kPtBlock), 0, st, mask, n, bits, cnt);
+  // every tile sums the counts before it, at most 8 loads a thread; beyond that
+  // the sums (quadratic in the tiles) cost more than a scan launch
+  const bool scan = nt > 8u * kPtBlock;
+  if (scan)
+    hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanThreads), 0, st, (const uint32_t *)nullptr, n, kCompactTile,
+                       (const uint32_t *)cnt, (const uint32_t *)nullptr, off, (uint32_t *)nullptr,
+                       (uint32_t *)nullptr, (uint32_t *)nullptr);
+  hipLaunchKernelGGL(k_compact_write, dim3(nt), dim3(kPtBlock), 0, st, mask, n, (const u64 *)bits,
+                     (const uint32_t *)cnt, scan ? (const uint32_t *)off : (const uint32_t *)nullptr, out_idx,
+                     out_count);
   return hipGetLastError();
 }
 
