@@ -92,15 +92,9 @@ __global__ void k_batch_init(uint32_t *queue, uint32_t first, uint32_t n, uint32
 hipError_t enqueue_spawn(const SpawnArgs &a, hipStream_t st) {
   if (a.slots == 0) return hipSuccess;
   const uint32_t grid = (a.slots + kBlock - 1) / kBlock;
-  uint32_t *cnt = a.blk, *off = a.blk + grid;
   hipLaunchKernelGGL(k_spawn, dim3(grid), dim3(kBlock), 0, st, a);
-  hipLaunchKernelGGL(compact::k_block_scan, dim3(1), dim3(compact::kScanThreads), 0, st, a.count_in, a.slots, kBlock,
-                     (const uint32_t *)cnt, (const uint32_t *)nullptr, off, (uint32_t *)nullptr, a.count_out,
-                     (uint32_t *)nullptr);
-  hipLaunchKernelGGL((compact::k_scatter2<kBlock>), dim3(grid), dim3(kBlock), 0, st, a.count_in, a.slots,
-                     (const uint32_t *)a.tmp, (const uint32_t *)nullptr, (const uint32_t *)cnt,
-                     (const uint32_t *)nullptr, (const uint32_t *)off, (const uint32_t *)nullptr, a.qout,
-                     (uint32_t *)nullptr, a.slots);
+  compact::enqueue_scatter<kBlock>(a.count_in, a.slots, a.tmp, nullptr, a.blk, grid, a.qout, nullptr, a.count_out,
+                                   nullptr, a.slots, st);
   return hipGetLastError();
 }
 

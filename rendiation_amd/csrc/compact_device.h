@@ -23,8 +23,9 @@ __device__ __forceinline__ uint32_t lane_rank(u64 m) {
 // 1. block_compact2 (inside the producing kernel): each block compacts its
 //    own items stably into tmp[bid * B + local rank] and writes its counts.
 // 2. k_block_scan: one workgroup turns the block counts into exclusive
-//    offsets and the totals.
-// 3. k_scatter2: each block copies its compacted run to out[offset + j].
+//    offsets and the totals; only for more than kDirectBlocks live blocks.
+// 3. k_scatter2: each block copies its compacted run to out[offset + j], its
+//    offset being the sum of the counts before it where there was no scan.
 // Block i holds the input slots [i * B, (i + 1) * B), so the output is a
 // stable copy_if whatever order the blocks run in.
 
@@ -59,6 +60,11 @@ __device__ __forceinline__ void block_compact2(bool ka, bool kb, uint32_t item, 
   }
 }
 
+// Live blocks whose offsets k_scatter2 sums itself: at most 16 loads a thread,
+// where the scan launch takes 7 to 9 us (a preview frame of 4 bounces: 431 ->
+// 395 us); beyond that the sums, quadratic in the blocks, cost more.
+constexpr uint32_t kDirectBlocks = 4096;
+
 constexpr uint32_t kScanThreads = 1024;
 constexpr uint32_t kScanPer = 8;                         // counts per thread per tile
 constexpr uint32_t kScanTile = kScanThreads * kScanPer;  // counts per tile
@@ -66,7 +72,8 @@ constexpr uint32_t kScanTile = kScanThreads * kScanPer;  // counts per tile
 namespace {
 
 // Exclusive scan of the block counts of the first ceil(min(*count_in,
-// slots) / B) blocks (one workgroup of kScanThreads): offsets and totals.
+// slots) / B) blocks (one workgroup of kScanThreads), when they are more than
+// `direct`: offsets and totals.
 // cnt_b / off_b / total_b may be null.  The counts stream through LDS in
 // tiles of kScanTile with coalesced loads and stores; each thread scans
 // kScanPer consecutive counts of a tile, the workgroup scans the thread sums,
@@ -74,11 +81,12 @@ namespace {
 __global__ __launch_bounds__(kScanThreads) void k_block_scan(const uint32_t *count_in, uint32_t slots, uint32_t B,
                                                              const uint32_t *cnt_a, const uint32_t *cnt_b,
                                                              uint32_t *off_a, uint32_t *off_b, uint32_t *total_a,
-                                                             uint32_t *total_b) {
+                                                             uint32_t *total_b, uint32_t direct) {
   __shared__ uint32_t t_a[kScanTile], t_b[kScanTile];
   __shared__ uint32_t s_a[kScanThreads / 64], s_b[kScanThreads / 64];
   const uint32_t n = count_in ? min(*count_in, slots) : slots;
   const uint32_t nb = (n + B - 1) / B;
+  if (direct && nb <= direct) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const bool two = cnt_b != nullptr;
   uint32_t carry_a = 0, carry_b = 0;
@@ -148,18 +156,72 @@ __global__ __launch_bounds__(kScanThreads) void k_block_scan(const uint32_t *cou
 }
 
 // Copies each block's compacted run to its offset (grid: one block of B
-// threads per possible input block; blocks past the live count return).
+// threads per possible input block; blocks past the live count return).  Up
+// to kDirectBlocks live blocks it sums the counts before its block itself and
+// its last live block writes the totals.
 template <int B>
 __global__ __launch_bounds__(B) void k_scatter2(const uint32_t *count_in, uint32_t slots, const uint32_t *tmp_a,
                                                 const uint32_t *tmp_b, const uint32_t *cnt_a, const uint32_t *cnt_b,
                                                 const uint32_t *off_a, const uint32_t *off_b, uint32_t *out_a,
-                                                uint32_t *out_b, uint32_t capacity) {
+                                                uint32_t *out_b, uint32_t *total_a, uint32_t *total_b,
+                                                uint32_t capacity) {
+  __shared__ uint32_t s_a, s_b;
   const uint32_t n = count_in ? min(*count_in, slots) : slots;
   const uint32_t nb = (n + B - 1) / B, bid = blockIdx.x, j = threadIdx.x;
-  if (bid >= nb) return;
+  if (bid >= nb) {
+    if (nb == 0 && bid == 0 && j == 0) {
+      if (total_a) *total_a = 0u;
+      if (total_b) *total_b = 0u;
+    }
+    return;
+  }
+  uint32_t at_a, at_b = 0;
+  if (nb <= kDirectBlocks) {
+    if (j == 0) s_a = s_b = 0u;
+    __syncthreads();
+    uint32_t a = 0, b = 0;
+    for (uint32_t t = j; t < bid; t += B) {
+      a += cnt_a[t];
+      if (cnt_b) b += cnt_b[t];
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      a += (uint32_t)__shfl_xor((int)a, o, 64);
+      b += (uint32_t)__shfl_xor((int)b, o, 64);
+    }
+    if ((j & 63u) == 0) {
+      if (a) atomicAdd(&s_a, a);
+      if (b) atomicAdd(&s_b, b);
+    }
+    __syncthreads();
+    at_a = s_a;
+    at_b = s_b;
+    if (bid + 1 == nb && j == 0) {
+      if (total_a) *total_a = at_a + cnt_a[bid];
+      if (total_b) *total_b = at_b + (cnt_b ? cnt_b[bid] : 0u);
+    }
+  } else {
+    at_a = off_a[bid];
+    if (cnt_b) at_b = off_b[bid];
+  }
   const size_t base = (size_t)bid * B;
-  if (j < cnt_a[bid] && off_a[bid] + j < capacity) out_a[off_a[bid] + j] = tmp_a[base + j];
-  if (cnt_b && j < cnt_b[bid] && off_b[bid] + j < capacity) out_b[off_b[bid] + j] = tmp_b[base + j];
+  if (j < cnt_a[bid] && at_a + j < capacity) out_a[at_a + j] = tmp_a[base + j];
+  if (cnt_b && j < cnt_b[bid] && at_b + j < capacity) out_b[at_b + j] = tmp_b[base + j];
+}
+
+// Passes 2 and 3: blk holds the counts of the one or two (tmp_b not null)
+// sets, `stride` words each, and room for their offsets.
+template <int B>
+void enqueue_scatter(const uint32_t *count_in, uint32_t slots, const uint32_t *tmp_a, const uint32_t *tmp_b,
+                     uint32_t *blk, uint32_t stride, uint32_t *out_a, uint32_t *out_b, uint32_t *total_a,
+                     uint32_t *total_b, uint32_t capacity, hipStream_t st) {
+  const uint32_t grid = (slots + B - 1) / B;
+  const uint32_t *cnt_a = blk, *cnt_b = tmp_b ? blk + stride : nullptr;
+  uint32_t *off_a = blk + (tmp_b ? 2u : 1u) * (size_t)stride, *off_b = tmp_b ? off_a + stride : nullptr;
+  if (grid > kDirectBlocks)
+    hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanThreads), 0, st, count_in, slots, (uint32_t)B, cnt_a, cnt_b,
+                       off_a, off_b, total_a, total_b, kDirectBlocks);
+  hipLaunchKernelGGL((k_scatter2<B>), dim3(grid), dim3(B), 0, st, count_in, slots, tmp_a, tmp_b, cnt_a, cnt_b,
+                     (const uint32_t *)off_a, (const uint32_t *)off_b, out_a, out_b, total_a, total_b, capacity);
 }
 
 }  // namespace

@@ -36,7 +36,6 @@ using pt::V3;
 using pt::v3;
 using compact::block_compact2;
 using compact::k_block_scan;
-using compact::k_scatter2;
 using compact::kScanThreads;
 using namespace pts;
 
@@ -246,7 +245,8 @@ __global__ __launch_bounds__(kPtBlock) void k_sum_visits(const uint32_t *queue, 
 // launch, which writes the indices in order, reads n / 8 bytes instead of it.
 // Bound by the launches at small n (n <= one tile: one launch) and by memory
 // at large n: 4.19M flags of 30 %, 22 MB in and out, 31 us with block-local
-// runs, a scan of 16k block counts and a copy; 14 us now.
+// runs, a scan of 16k block counts and a copy; 10.9 us now
+// (3.8 and 6.2 us of kernels).
 constexpr uint32_t kCompactRows = 16;
 static_assert(kCompactTile == kPtBlock * kCompactRows, "a row per wave and step");
 
@@ -486,16 +486,12 @@ __global__ void k_sobol(const uint32_t *index, const uint32_t *scr, uint32_t n, 
   out[2 * i + 1] = pt::sobol1(index[i], scr[2 * i + 1]);
 }
 
-// Scan of the shade kernel's block counts and scatter into the next
-// extension queue and the shadow queue (sizes to counts[b + 1] and
-// counts[max_bounces + 2 + b]).
-void enqueue_queue_scatter(const PtLaunch &P, uint32_t b, uint32_t grid, hipStream_t st) {
-  uint32_t *qout = (b & 1) ? P.qa : P.qb;
-  const uint32_t s = P.blk_stride;
-  hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanThreads), 0, st, P.counts + b, P.npaths, kPtBlock, P.blk,
-                     P.blk + s, P.blk + 2 * s, P.blk + 3 * s, P.counts + b + 1, P.counts + P.max_bounces + 2 + b);
-  hipLaunchKernelGGL((k_scatter2<kPtBlock>), dim3(grid), dim3(kPtBlock), 0, st, P.counts + b, P.npaths, P.tmp_a,
-                     P.tmp_b, P.blk, P.blk + s, P.blk + 2 * s, P.blk + 3 * s, qout, P.qs, P.npaths);
+// The shade kernel's runs into the next extension queue and the shadow queue
+// (sizes to counts[b + 1] and counts[max_bounces + 2 + b]).
+void enqueue_queue_scatter(const PtLaunch &P, uint32_t b, hipStream_t st) {
+  compact::enqueue_scatter<kPtBlock>(P.counts + b, P.npaths, P.tmp_a, P.tmp_b, P.blk, P.blk_stride,
+                                     (b & 1) ? P.qa : P.qb, P.qs, P.counts + b + 1, P.counts + P.max_bounces + 2 + b,
+                                     P.npaths, st);
 }
 
 }  // namespace
@@ -570,7 +566,7 @@ hipError_t enqueue_pt_frame(const PtLaunch &P, const TraceParams &scene, uint32_
   if (e != hipSuccess) return e;
   for (uint32_t b = 0; b <= P.max_bounces; b++) {
     hipLaunchKernelGGL((k_pt_shade<kPtBlock, false>), dim3(grid), dim3(kPtBlock), 0, st, P, b);
-    enqueue_queue_scatter(P, b, grid, st);
+    enqueue_queue_scatter(P, b, st);
     if (b == P.max_bounces) break;
     if (P.tail_b0 && b == P.tail_b0 && !count) {
       // one launch finishes every path from here (its shadow ray of bounce b on)
@@ -638,7 +634,7 @@ hipError_t enqueue_pt_replay(const PtLaunch &P, const TraceParams &scene, uint32
     e = launch_trace(tp, RDRT_TRAVERSAL_FAST, push_depth, tune, st);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_pt_shade<kPtBlock, true>), dim3(grid), dim3(kPtBlock), 0, st, P, b);
-    enqueue_queue_scatter(P, b, grid, st);
+    enqueue_queue_scatter(P, b, st);
   }
   // each record adds to at most 3 entries of one vertex component
   e = det::enqueue_scale(db.h, 3ull * P.max_bounces * P.npaths, st);
@@ -718,7 +714,7 @@ hipError_t enqueue_compact(const uint32_t *mask, uint32_t n, uint32_t *out_idx, 
   if (scan)
     hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanThreads), 0, st, (const uint32_t *)nullptr, n, kCompactTile,
                        (const uint32_t *)cnt, (const uint32_t *)nullptr, off, (uint32_t *)nullptr,
-                       (uint32_t *)nullptr, (uint32_t *)nullptr);
+                       (uint32_t *)nullptr, (uint32_t *)nullptr, 0u);
   hipLaunchKernelGGL(k_compact_write, dim3(nt), dim3(kPtBlock), 0, st, mask, n, (const u64 *)bits,
                      (const uint32_t *)cnt, scan ? (const uint32_t *)off : (const uint32_t *)nullptr, out_idx,
                      out_count);

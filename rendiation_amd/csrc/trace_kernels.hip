@@ -153,13 +153,8 @@ hipError_t enqueue_cull(const TraceParams &p, const CullScratch &cs, hipStream_t
   if (p.queue || p.count) return hipErrorInvalidValue;
   const uint32_t nb = (p.n + kCullBlock - 1) / kCullBlock;
   hipLaunchKernelGGL(k_trace_cull, dim3(nb), dim3(kCullBlock), 0, st, p, cs);
-  hipLaunchKernelGGL(compact::k_block_scan, dim3(1), dim3(compact::kScanThreads), 0, st, (const uint32_t *)nullptr,
-                     p.n, kCullBlock, (const uint32_t *)cs.blk, (const uint32_t *)nullptr, cs.blk + nb,
-                     (uint32_t *)nullptr, cs.count, (uint32_t *)nullptr);
-  hipLaunchKernelGGL((compact::k_scatter2<kCullBlock>), dim3(nb), dim3(kCullBlock), 0, st, (const uint32_t *)nullptr,
-                     p.n, (const uint32_t *)cs.tmp, (const uint32_t *)nullptr, (const uint32_t *)cs.blk,
-                     (const uint32_t *)nullptr, (const uint32_t *)(cs.blk + nb), (const uint32_t *)nullptr, cs.queue,
-                     (uint32_t *)nullptr, p.n);
+  compact::enqueue_scatter<kCullBlock>(nullptr, p.n, cs.tmp, nullptr, cs.blk, nb, cs.queue, nullptr, cs.count, nullptr,
+                                       p.n, st);
   return hipGetLastError();
 }
 
