@@ -111,7 +111,7 @@ struct Dev {
   float *na, *ns;      // bin origin and step (reference) or centre min and scale (fast)
   u32 *nbest;          // fast: best bin
   u32 *nright, *ngeo;  // right-child steps on the path from the root; geometry
-  u32 *count;          // [0] node count, [1] median splits this level, [2] error bits
+  u32 *count;          // [0] node count, [1] median splits this level, [2] error bits, [3] next level's begin
   u32 cap;             // node capacity
   // per active slot
   u32 *cb;             // 6 keys per slot (centre bounds, fast)
@@ -159,6 +159,33 @@ __global__ __launch_bounds__(kB) void k_centres(Dev d, const u32 *geo_of) {
   d.node_of[i] = geo_of[i];
 }
 
+// Folds the lanes' keys c (3 minima, 3 maxima) into keys[6 * slot]: a wave
+// meets few nodes, whose ranges are contiguous, so each node's lanes are
+// reduced in registers and 6 lanes add the result.  An atomic per lane and key
+// made k_centre_bounds 100 us on a level of 100k triangles (LDS words where a
+// block had one node); 7 us now.  Whole waves call this (slot kInvalid:
+// nothing to add).
+__device__ __forceinline__ void fold_keys(u32 *keys, u32 slot, const u32 c[6]) {
+  const u32 lane = threadIdx.x & 63u;
+  unsigned long long todo = __ballot(slot != kInvalid);
+  while (todo) {
+    const u32 of = (u32)__shfl((int)slot, __ffsll(todo) - 1, 64);
+    const bool mine = slot == of;
+    todo &= ~__ballot(mine);
+    u32 out = 0;
+    for (u32 k = 0; k < 6; k++) {
+      u32 v = mine ? c[k] : k < 3 ? kMinInit : kMaxInit;
+      for (int o = 32; o > 0; o >>= 1) {
+        const u32 w = (u32)__shfl_xor((int)v, o, 64);
+        v = k < 3 ? min(v, w) : max(v, w);
+      }
+      if (lane == k) out = v;
+    }
+    if (lane < 3) atomicMin(&keys[6 * (size_t)of + lane], out);
+    else if (lane < 6) atomicMax(&keys[6 * (size_t)of + lane], out);
+  }
+}
+
 // Union of the primitive boxes of every active node flagged `want` (1 =
 // all, 2 = children of median splits, whose boxes are range unions), into
 // nbox as keys first (nbox reinterpreted), decoded by k_decode_boxes.
@@ -168,24 +195,19 @@ __global__ __launch_bounds__(kB) void k_range_boxes(Dev d, u32 *keys) {
   if (nd_block != kInvalid && threadIdx.x < 6) s[threadIdx.x] = threadIdx.x < 3 ? kMinInit : kMaxInit;
   __syncthreads();
   const u32 i = blockIdx.x * kB + threadIdx.x;
+  u32 slot = kInvalid, c[6] = {};
   if (i < d.n) {
     const u32 nd = d.node_of[i];
     if (active(d, nd)) {
       const DBox b = prim_box(d, d.order[i]);
-      if (nd_block != kInvalid) {
-        for (int k = 0; k < 3; k++) {
-          atomicMin(&s[k], fkey(b.mn[k]));
-          atomicMax(&s[3 + k], fkey(b.mx[k]));
-        }
-      } else {
-        u32 *q = keys + 6 * (size_t)(nd - d.lo);
-        for (int k = 0; k < 3; k++) {
-          atomicMin(&q[k], fkey(b.mn[k]));
-          atomicMax(&q[3 + k], fkey(b.mx[k]));
-        }
+      slot = nd_block != kInvalid ? 0u : nd - d.lo;
+      for (int k = 0; k < 3; k++) {
+        c[k] = fkey(b.mn[k]);
+        c[3 + k] = fkey(b.mx[k]);
       }
     }
   }
+  fold_keys(nd_block != kInvalid ? s : keys, slot, c);
   __syncthreads();
   if (nd_block != kInvalid && threadIdx.x < 6) {
     u32 *q = keys + 6 * (size_t)(nd_block - d.lo);
@@ -211,18 +233,16 @@ __global__ __launch_bounds__(kB) void k_centre_bounds(Dev d) {
   if (nd_block != kInvalid && threadIdx.x < 6) s[threadIdx.x] = threadIdx.x < 3 ? kMinInit : kMaxInit;
   __syncthreads();
   const u32 i = blockIdx.x * kB + threadIdx.x;
+  u32 slot = kInvalid, c[6] = {};
   if (i < d.n) {
     const u32 nd = d.node_of[i];
     if (active(d, nd)) {
       const u32 p = d.order[i];
-      u32 *q = nd_block != kInvalid ? s : d.cb + 6 * (size_t)(nd - d.lo);
-      for (int k = 0; k < 3; k++) {
-        const u32 c = fkey(d.cen[3 * (size_t)p + k]);
-        atomicMin(&q[k], c);
-        atomicMax(&q[3 + k], c);
-      }
+      slot = nd_block != kInvalid ? 0u : nd - d.lo;
+      for (int k = 0; k < 3; k++) c[k] = c[3 + k] = fkey(d.cen[3 * (size_t)p + k]);
     }
   }
+  fold_keys(nd_block != kInvalid ? s : d.cb, slot, c);
   __syncthreads();
   if (nd_block != kInvalid && threadIdx.x < 6) {
     u32 *q = d.cb + 6 * (size_t)(nd_block - d.lo);
@@ -237,6 +257,7 @@ __global__ __launch_bounds__(kB) void k_centre_bounds(Dev d) {
 __global__ void k_prep(Dev d) {
   const u32 j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= d.m) return;
+  if (j == 0) d.count[3] = d.count[0];  // k_small's nodes end here: the next level begins
   const u32 nd = d.lo + j;
   if (d.nflags[nd] & kDone) return;
   if (d.mode == 0) {
@@ -939,6 +960,7 @@ __global__ void k_roots(Dev d, const u32 *off, u32 ngeo) {
     d.count[0] = ngeo;
     d.count[1] = 0u;
     d.count[2] = 0u;
+    d.count[3] = ngeo;
   }
   if (g >= ngeo) return;
   d.nbeg[g] = off[g];
@@ -1151,18 +1173,19 @@ class Builder final : public DeviceTreeBuilder {
       hipLaunchKernelGGL(k_scan_apply, dim3(sb), dim3(kB), 0, st_, d);
       hipLaunchKernelGGL(k_scatter, dim3(g), dim3(kB), 0, st_, d);
       DB_TRY(hipGetLastError());
-      u32 counts[3];
-      DB_TRY(hipMemcpyAsync(counts, d.count, 12, hipMemcpyDeviceToHost, st_));
+      u32 counts[4];
+      DB_TRY(hipMemcpyAsync(counts, d.count, 16, hipMemcpyDeviceToHost, st_));
       DB_TRY(hipStreamSynchronize(st_));
       if (counts[2]) {
         error_ = counts[2] & kErrMedian ? "a median split of more than 4096 primitives (reference tree)"
                                         : "more nodes than 2n + 1 per geometry (bin_size 0)";
         return hipErrorNotSupported;
       }
-      const u32 made = counts[0] - total;
+      // the nodes that k_small made are finished: no level of theirs
+      const u32 next = counts[3], made = counts[0] - next;
       if (counts[1]) {  // children of median splits: boxes are the unions of their ranges
         Dev c = d;
-        c.lo = total;
+        c.lo = next;
         c.m = made;
         c.node_of = d.node_of2;
         c.order = d.order2;
@@ -1174,7 +1197,7 @@ class Builder final : public DeviceTreeBuilder {
       }
       std::swap(d.order, d.order2);
       std::swap(d.node_of, d.node_of2);
-      lo = total;
+      lo = next;
       m = made;
       total = counts[0];
       hipLaunchKernelGGL(k_reset_counts, dim3(1), dim3(1), 0, st_, d.count, total);
