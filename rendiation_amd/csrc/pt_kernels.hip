@@ -11,11 +11,10 @@
 // Queue sizes stay on the device, so a whole frame is one capturable
 // sequence with no host round trip.
 //
-// Compaction: one pass fused into the shade kernel.  Each wave ballots its
-// keep flags (rank = mbcnt), each block sums its waves in LDS and gets its
-// exclusive offset by decoupled look-back over per-block status words; block
-// order comes from an atomic ticket, so every predecessor a block waits on
-// is already running.  The output equals a stable copy_if
+// Compaction: its first pass is fused into the shade kernel.  Each wave ballots
+// its keep flags (rank = mbcnt), each block sums its waves in LDS and writes a
+// run and its length; a scatter launch copies the runs to their offsets.  No
+// block waits for another, and the output equals a stable copy_if
 // (shader/parallel-compute/src/stream_compaction.rs:3-45).
 
 #include <algorithm>
