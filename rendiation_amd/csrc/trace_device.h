@@ -16,28 +16,32 @@
 //    their own front to back, with a per-lane stack in LDS (column layout
 //    [entry][lane]: each lane owns one bank at every depth, so stack traffic
 //    is conflict-free), and test triangles from 64-byte pre-pass records with
-//    the reference's arithmetic, so t, u, v are bit-identical.  Their node
-//    tests are fused multiply-adds widened by their rounding error: they may
-//    pass a box that the reference's test fails, never the other way round.
-//    Only the visit order differs, which can change the winner among hits with
-//    equal t.
+//    the reference's arithmetic, so t, u, v are bit-identical.  Their box tests
+//    are the reference's too (box_test.h), so child pairs and child quads,
+//    which hold the same leaf boxes, report a hit for the same rays, and only
+//    the visit order differs, which can change the winner among hits with
+//    equal t.  Quantized quads widen the boxes to 8-bit planes: a ray that
+//    passes a leaf's box by less than a plane's step may hit with them only.
 //
 //    What bounded these kernels was idle lanes: with every lane doing whatever
 //    it was at, 9 (1M rays in 100k triangles) to 15 (height field, first
 //    bounce) of 64 lanes worked per vector instruction.  trace_wave gives the
-//    wave one kind of work at a time and refills it: 19 to 30 lanes.  With the
-//    node tests in fewer instructions, no round trip to memory behind them and
-//    a work counter per XCD, 1M rays went from 0.487 to 0.337 ms, the 1080p
-//    frame from 2.39 to 1.85 ms, a height-field step of 16 views from 24.7 to
-//    20.8 ms, a batch of 16 scenes from 4.33 to 2.31 ms.
+//    wave one kind of work at a time and refills it.  With near and far planes
+//    chosen by the loads, no round trip to memory behind the node tests and a
+//    work counter per XCD, 1M rays went from 0.49 to 0.35 ms, the 1080p frame
+//    from 2.4 to 1.8 ms, a height-field step of 16 views from 24.7 to 20.8 ms,
+//    a batch of 16 scenes from 4.3 to 2.4 ms.  (A fused multiply-add per plane
+//    would make that 0.33, 1.7 and 2.3 ms, but it loses hits: box_test.h.)
 //
 // Compiled with -ffp-contract=off and IEEE division/sqrt: one rounding per
-// operation, as in the reference, but for the node tests.
+// operation, as in the reference.
 #ifndef RDRT_TRACE_DEVICE_H
 #define RDRT_TRACE_DEVICE_H
 
 #include <algorithm>
+#include <type_traits>
 
+#include "box_test.h"
 #include "trace_kernels.h"
 
 #pragma clang fp contract(off)
@@ -50,9 +54,6 @@ constexpr uint32_t F_FORCE_OPAQUE = 0x01, F_FORCE_NON_OPAQUE = 0x02, F_END_SEARC
                    F_SKIP_TRIANGLES = 0x100, F_FLIP = 0x400;
 constexpr uint32_t GI_CULL_DISABLE = 0x1, GI_FLIP = 0x2, GI_FORCE_OPAQUE = 0x4, GI_FORCE_NO_OPAQUE = 0x8;
 
-struct F3 {
-  float x, y, z;
-};
 __device__ __forceinline__ F3 f3(float x, float y, float z) { return F3{x, y, z}; }
 __device__ __forceinline__ F3 sub(F3 a, F3 b) { return f3(a.x - b.x, a.y - b.y, a.z - b.z); }
 __device__ __forceinline__ float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
@@ -68,20 +69,6 @@ __device__ __forceinline__ F3 normalize(F3 a) {
   return a;
 }
 __device__ __forceinline__ F3 recip(F3 a) { return f3(1.0f / a.x, 1.0f / a.y, 1.0f / a.z); }
-
-// Ray/AABB slab test (wavefront_compute/geometry/mod.rs:44-64).  inv_d is
-// 1/dir, hoisted out of the node loop; the per-node values are unchanged.
-__device__ __forceinline__ bool slab(F3 o, F3 inv_d, float tmin, float tmax, float mnx, float mny, float mnz,
-                                     float mxx, float mxy, float mxz, float &tnear) {
-  float t0x = (mnx - o.x) * inv_d.x, t0y = (mny - o.y) * inv_d.y, t0z = (mnz - o.z) * inv_d.z;
-  float t1x = (mxx - o.x) * inv_d.x, t1y = (mxy - o.y) * inv_d.y, t1z = (mxz - o.z) * inv_d.z;
-  float nx = fminf(t0x, t1x), ny = fminf(t0y, t1y), nz = fminf(t0z, t1z);
-  float fx = fmaxf(t0x, t1x), fy = fmaxf(t0y, t1y), fz = fmaxf(t0z, t1z);
-  float tn = fmaxf(fmaxf(nx, ny), nz);
-  float tf = fminf(fminf(fx, fy), fz);
-  tnear = tn;
-  return tn <= tf && tmin < tf && tn < tmax;
-}
 
 // Triangle test given the vertex-only quantities (geometry/mod.rs:118-154).
 // b == 0 is a miss.
@@ -240,56 +227,14 @@ struct Kids {
   uint32_t n, r[4];
 };
 
-// A ray as the node tests take it: per axis 1 / dir and the constants of
-// t = plane * inv + bias for the near and the far planes.  The fused form
-// takes half the instructions of (plane - o) * inv; its rounding error against
-// that form is that of o * inv, at most 2^-23 |o * inv|, which the biases
-// move outwards, so a node test may pass a box that the exact test fails,
-// never the other way round.  |inv| is bounded (2^60), so that an axis-parallel
-// ray gets large finite distances and no NaN on that axis.
-//
-// The child-pair layout keeps the reference's arithmetic, (plane - o) * inv
-// (RayBox::nb is the origin there, fb unused): its two tests gain nothing from
-// the fused form, and on grids of axis-aligned edges the exact form decides
-// thousands of rays that pass within rounding of an edge.
-struct RayBox {
-  F3 inv, nb, fb;
-};
-__device__ __forceinline__ void ray_box_axis(float o, float inv, float &iv, float &nb, float &fb) {
-  constexpr float kMost = 1.152921504606846976e18f, kErr = 2.384185791015625e-7f;  // 2^60, 2^-22
-  iv = fminf(fmaxf(inv, -kMost), kMost);
-  const float c = -(o * iv), e = fabsf(c) * kErr;
-  nb = c - e;
-  fb = c + e;
-}
-template <int LAYOUT>
-__device__ __forceinline__ RayBox ray_box(F3 o, F3 inv) {
-  RayBox r;
-  if constexpr (LAYOUT == 0) return RayBox{inv, o, f3(0.0f, 0.0f, 0.0f)};
-  ray_box_axis(o.x, inv.x, r.inv.x, r.nb.x, r.fb.x);
-  ray_box_axis(o.y, inv.y, r.inv.y, r.nb.y, r.fb.y);
-  ray_box_axis(o.z, inv.z, r.inv.z, r.nb.z, r.fb.z);
-  return r;
-}
 __device__ __forceinline__ bool negative(float v) { return (__float_as_uint(v) & 0x80000000u) != 0u; }
-
-// Near and far planes (already chosen by the direction's sign) of one box.
-__device__ __forceinline__ bool box_hit(const RayBox &r, float tmin, float tmax, float nx, float ny, float nz, float fx,
-                                        float fy, float fz, float &tnear) {
-  const float tn = fmaxf(fmaxf(__builtin_fmaf(nx, r.inv.x, r.nb.x), __builtin_fmaf(ny, r.inv.y, r.nb.y)),
-                         __builtin_fmaf(nz, r.inv.z, r.nb.z));
-  const float tf = fminf(fminf(__builtin_fmaf(fx, r.inv.x, r.fb.x), __builtin_fmaf(fy, r.inv.y, r.fb.y)),
-                         __builtin_fmaf(fz, r.inv.z, r.fb.z));
-  tnear = tn;
-  return tn <= tf && tmin < tf && tn < tmax;
-}
 
 __device__ __forceinline__ Kids kids_pair(const PairNode *node, const RayBox &r, float tmin, float tmax) {
   const float4 *q = reinterpret_cast<const float4 *>(node);
   const float4 a = q[0], b = q[1], c = q[2], d = q[3];
   float tl, tr;
-  const bool hl = slab(r.nb, r.inv, tmin, tmax, a.x, a.y, a.z, b.x, b.y, b.z, tl);
-  const bool hr = slab(r.nb, r.inv, tmin, tmax, c.x, c.y, c.z, d.x, d.y, d.z, tr);
+  const bool hl = slab(r.o, r.inv, tmin, tmax, a.x, a.y, a.z, b.x, b.y, b.z, tl);
+  const bool hr = slab(r.o, r.inv, tmin, tmax, c.x, c.y, c.z, d.x, d.y, d.z, tr);
   const uint32_t lref = __float_as_uint(a.w), rref = __float_as_uint(c.w);
   const bool rlast = hr && (!hl || tr < tl);  // the right child is the nearest hit
   Kids k;
@@ -337,6 +282,7 @@ __device__ __forceinline__ Kids sort_kids(const bool h[4], const float t[4], uin
   return k;
 }
 
+template <bool PLAIN>
 __device__ __forceinline__ Kids kids_quad(const QuadNode *node, const RayBox &r, float tmin, float tmax) {
   // the rows of the near and the far planes of an axis swap with the
   // direction's sign: 16 bytes apart, so the loads pick them
@@ -351,21 +297,14 @@ __device__ __forceinline__ Kids kids_quad(const QuadNode *node, const RayBox &r,
   const uint4 rf = *reinterpret_cast<const uint4 *>(q + 96);
   float t[4];
   bool h[4];
-  h[0] = box_hit(r, tmin, tmax, xn.x, yn.x, zn.x, xf.x, yf.x, zf.x, t[0]);
-  h[1] = box_hit(r, tmin, tmax, xn.y, yn.y, zn.y, xf.y, yf.y, zf.y, t[1]);  // slots 0, 1 always used
-  h[2] = box_hit(r, tmin, tmax, xn.z, yn.z, zn.z, xf.z, yf.z, zf.z, t[2]) && rf.z != kInvalid;
-  h[3] = box_hit(r, tmin, tmax, xn.w, yn.w, zn.w, xf.w, yf.w, zf.w, t[3]) && rf.w != kInvalid;
+  h[0] = planes_hit<PLAIN>(r, tmin, tmax, xn.x, yn.x, zn.x, xf.x, yf.x, zf.x, t[0]);
+  h[1] = planes_hit<PLAIN>(r, tmin, tmax, xn.y, yn.y, zn.y, xf.y, yf.y, zf.y, t[1]);  // slots 0, 1 always used
+  h[2] = planes_hit<PLAIN>(r, tmin, tmax, xn.z, yn.z, zn.z, xf.z, yf.z, zf.z, t[2]) && rf.z != kInvalid;
+  h[3] = planes_hit<PLAIN>(r, tmin, tmax, xn.w, yn.w, zn.w, xf.w, yf.w, zf.w, t[3]) && rf.w != kInvalid;
   return sort_kids(h, t, rf);
 }
 
-// Quantized planes: corner + q * step, so t = q * (step * inv) + (corner *
-// inv + bias): two instructions per plane (byte to float, fused multiply-add).
-// The rounding of step * inv, at most 255 * 2^-24 of it, moves the bias
-// outwards too.
-__device__ __forceinline__ float quant_t(uint32_t word, int c, float step, float base) {
-  return __builtin_fmaf((float)((word >> (8 * c)) & 0xffu), step, base);
-}
-
+template <bool PLAIN>
 __device__ __forceinline__ Kids kids_qquad(const QuadNodeQ *node, const RayBox &r, float tmin, float tmax) {
   const float4 *q = reinterpret_cast<const float4 *>(node);
   const float4 a = q[0];                                  // corner, x step
@@ -376,33 +315,23 @@ __device__ __forceinline__ Kids kids_qquad(const QuadNodeQ *node, const RayBox &
   const bool sx = negative(r.inv.x), sy = negative(r.inv.y), sz = negative(r.inv.z);
   const uint32_t nx = sx ? xy.y : xy.x, fx = sx ? xy.x : xy.y, ny = sy ? xy.w : xy.z, fy = sy ? xy.z : xy.w,
                  nz = sz ? hiz : loz, fz = sz ? loz : hiz;
-  constexpr float kErr = 6.103515625e-5f;  // 2^-14 > 255 * 2^-23
-  const float ax = a.w * r.inv.x, ay = zs.z * r.inv.y, az = zs.w * r.inv.z;
-  const float bnx = __builtin_fmaf(fabsf(ax), -kErr, __builtin_fmaf(a.x, r.inv.x, r.nb.x)),
-              bny = __builtin_fmaf(fabsf(ay), -kErr, __builtin_fmaf(a.y, r.inv.y, r.nb.y)),
-              bnz = __builtin_fmaf(fabsf(az), -kErr, __builtin_fmaf(a.z, r.inv.z, r.nb.z)),
-              bfx = __builtin_fmaf(fabsf(ax), kErr, __builtin_fmaf(a.x, r.inv.x, r.fb.x)),
-              bfy = __builtin_fmaf(fabsf(ay), kErr, __builtin_fmaf(a.y, r.inv.y, r.fb.y)),
-              bfz = __builtin_fmaf(fabsf(az), kErr, __builtin_fmaf(a.z, r.inv.z, r.fb.z));
   float t[4];
   bool h[4];
 #pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const float tn = fmaxf(fmaxf(quant_t(nx, c, ax, bnx), quant_t(ny, c, ay, bny)), quant_t(nz, c, az, bnz));
-    const float tf = fminf(fminf(quant_t(fx, c, ax, bfx), quant_t(fy, c, ay, bfy)), quant_t(fz, c, az, bfz));
-    t[c] = tn;
-    h[c] = tn <= tf && tmin < tf && tn < tmax;
-  }
+  for (int c = 0; c < 4; c++)
+    h[c] = planes_hit<PLAIN>(r, tmin, tmax, dequant(a.x, nx, c, a.w), dequant(a.y, ny, c, zs.z),
+                             dequant(a.z, nz, c, zs.w), dequant(a.x, fx, c, a.w), dequant(a.y, fy, c, zs.z),
+                             dequant(a.z, fz, c, zs.w), t[c]);
   h[2] = h[2] && rf.z != kInvalid;  // slots 0, 1 always used
   h[3] = h[3] && rf.w != kInvalid;
   return sort_kids(h, t, rf);
 }
 
-template <int LAYOUT>
+template <int LAYOUT, bool PLAIN>
 __device__ __forceinline__ Kids test_kids(const TraceParams &p, bool world, uint32_t ref, const RayBox &r, float tmin,
                                           float tmax) {
-  if constexpr (LAYOUT == 2) return kids_qquad((world ? p.tlas_qquads : p.tri_qquads) + ref, r, tmin, tmax);
-  else if constexpr (LAYOUT == 1) return kids_quad((world ? p.tlas_quads : p.tri_quads) + ref, r, tmin, tmax);
+  if constexpr (LAYOUT == 2) return kids_qquad<PLAIN>((world ? p.tlas_qquads : p.tri_qquads) + ref, r, tmin, tmax);
+  else if constexpr (LAYOUT == 1) return kids_quad<PLAIN>((world ? p.tlas_quads : p.tri_quads) + ref, r, tmin, tmax);
   else return kids_pair((world ? p.tlas_pairs : p.tri_pairs) + ref, r, tmin, tmax);
 }
 
@@ -544,6 +473,14 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
     return load_ray(q, rid);
   };
 
+  auto node_step = [&](auto plain) {
+    const bool world = (st & kStWorld) != 0u;
+    if constexpr (CNT) cn += world ? 0u : 1u;
+    const float fs = far_ * s;
+    ref = stk.template step<LAYOUT>(
+        [&]() { return test_kids<LAYOUT, decltype(plain)::value>(p, world, ref, box, near_, fs); });
+  };
+
   for (;;) {
     const uint32_t idle = wave_count(ref == kRefDone);
     if (idle == 64u || (!last && idle >= kRefill)) {
@@ -583,7 +520,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
         if (rid < p.n) {  // a queue entry always names one of the n rays
           const RayIn r = ray_of();
           const F3 winv = recip(r.d);
-          box = ray_box<LAYOUT>(r.o, winv);
+          box = ray_box(r.o, winv);
           near_ = r.tmin;
           far_ = r.tmax;
           s = 1.0f;
@@ -606,15 +543,19 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
     }
     uint32_t a = wave_count(ref < kRefExit);
     if (a * kKeep >= 64u - idle) {
-      do {
-        if (ref < kRefExit) {
-          const bool world = (st & kStWorld) != 0u;
-          if constexpr (CNT) cn += world ? 0u : 1u;
-          const float fs = far_ * s;
-          ref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, world, ref, box, near_, fs); });
-        }
-        a = wave_count(ref < kRefExit);
-      } while (a * kKeep >= 64u - idle);
+      // the steps leave `box` as it is: which test they take is decided once
+      const bool plain = LAYOUT == 0 || __ballot(ref < kRefExit && !box.plain) == 0ull;
+      if (plain) {
+        do {
+          if (ref < kRefExit) node_step(std::true_type{});
+          a = wave_count(ref < kRefExit);
+        } while (a * kKeep >= 64u - idle);
+      } else {
+        do {
+          if (ref < kRefExit) node_step(std::false_type{});
+          a = wave_count(ref < kRefExit);
+        } while (a * kKeep >= 64u - idle);
+      }
       continue;
     }
     const bool leaf = (ref & kLeafBit) != 0u, world = (st & kStWorld) != 0u;
@@ -688,7 +629,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
                  (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) | ((fl & F_END_SEARCH) ? kStEnd : 0u) |
                  (g + 1u < gend ? kStGeometries : 0u) | (left << kStMoreShift);
             geo = g;
-            box = ray_box<LAYOUT>(o, inv);
+            box = ray_box(o, inv);
             stk.push(kRefExit);  // the end mark of the BLAS, above the TLAS entries
             ref = LAYOUT ? gr.quad_root : gr.root_ref;
             break;
@@ -697,7 +638,7 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
           continue;
         }
         if (left == 0u) {
-          box = ray_box<LAYOUT>(r.o, winv);
+          box = ray_box(r.o, winv);
           near_ = r.tmin;
           s = 1.0f;
           st |= kStWorld;
@@ -791,6 +732,15 @@ __device__ __forceinline__ bool group_any(bool b) {
 // kCoopHit when the ray hit.
 constexpr uint32_t kCoopHit = 0x100u;
 
+// The step of the lanes at an inner node.
+template <int LAYOUT, class Stack>
+__device__ __forceinline__ uint32_t inner_step(Stack &stk, const TraceParams &p, bool world, uint32_t ref,
+                                               const RayBox &box, float tmin, float tmax) {
+  if (LAYOUT == 0 || __ballot(!box.plain) == 0ull)  // wave-uniform
+    return stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT, true>(p, world, ref, box, tmin, tmax); });
+  return stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT, false>(p, world, ref, box, tmin, tmax); });
+}
+
 template <int K, int S, int B, int LAYOUT, int G = (int)kCoopLanes>
 __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_t rid, uint32_t *lds,
                                                    uint32_t glane) {
@@ -836,7 +786,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
         cull_triangle(fl, ce, cb);
         st = (geometry_opaque(fl, geo.flags) ? kStOpaque : 0u) | (ce ? kStCull : 0u) | (cb ? kStCullBack : 0u) |
              ((fl & F_END_SEARCH) ? kStEnd : 0u);
-        box = ray_box<LAYOUT>(bo, binv);
+        box = ray_box(bo, binv);
         stk.push(kRefExit);  // above the TLAS entries
         bref = LAYOUT ? geo.quad_root : geo.root_ref;
         break;
@@ -847,8 +797,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
       const uint32_t a = wave_count(bref < kRefExit), b = wave_count((bref & kLeafBit) != 0u);
       if (a + b == 0u) break;
       if (a * kCoopKeep >= a + b) {
-        if (bref < kRefExit)
-          bref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, false, bref, box, near_s, far_ * s); });
+        if (bref < kRefExit) bref = inner_step<LAYOUT>(stk, p, false, bref, box, near_s, far_ * s);
       } else if (bref & kLeafBit) {
         const uint32_t k0 = (bref & ~kLeafBit) >> kLeafCountBits, k1 = k0 + (bref & kLeafMaxCount);
         F3 bo, bd;
@@ -906,10 +855,10 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
                    root->mx[2], tn)) {
     uint32_t ref = LAYOUT ? p.tlas_quad_roots[root - p.tlas_roots] : root->root_ref;
     stk.push(kRefDone);
-    RayBox box = ray_box<LAYOUT>(r.o, winv);
+    RayBox box = ray_box(r.o, winv);
     while (ref != kRefDone) {
       if (!(ref & kLeafBit)) {
-        ref = stk.template step<LAYOUT>([&]() { return test_kids<LAYOUT>(p, true, ref, box, r.tmin, far_); });
+        ref = inner_step<LAYOUT>(stk, p, true, ref, box, r.tmin, far_);
       } else {
         const uint32_t i0 = (ref & ~kLeafBit) >> kLeafCountBits, i1 = i0 + (ref & kLeafMaxCount);
         for (uint32_t i = i0; i < i1 && !done; i++) {
@@ -923,7 +872,7 @@ __device__ __forceinline__ uint32_t trace_coop_one(const TraceParams &p, uint32_
           if (++cnt == (uint32_t)G) {
             flush();
             winv = recip(r.d);
-            box = ray_box<LAYOUT>(r.o, winv);
+            box = ray_box(r.o, winv);
           }
         }
         if (done) break;
