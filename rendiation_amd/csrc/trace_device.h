@@ -363,7 +363,8 @@ struct LaneStack {
     o = f3(q[0], q[B], q[2 * B]);
     d = f3(q[3 * B], q[4 * B], q[5 * B]);
   }
-  __device__ __forceinline__ bool deep() const { return sp + 3u > R; }
+  // near the end of the LDS rows, or of the stack: put() spills, or drops and reports
+  __device__ __forceinline__ bool deep() const { return sp + 3u > (R < N ? R : N); }
   __device__ __forceinline__ uint32_t get(uint32_t i) const {
     if (N <= R || i < R) return lds[i * B];
     uint32_t v = spill[i - R];

@@ -1,5 +1,6 @@
-"""Builds tests/stages/libpipeline_stages.so, the stage kernels of the
-pipeline tests, with the library's own compiler flags."""
+"""Builds the device code that only tests run, with the library's own compiler
+flags: tests/stages/libpipeline_stages.so, the stage kernels of the pipeline
+tests, and tests/stages/libstack_stages.so, the traversal's stack alone."""
 
 from __future__ import annotations
 
@@ -18,9 +19,10 @@ def build() -> Path:
     from rendiation_amd import build as rb
 
     hipcc = rb._hipcc()
-    tmp = LIB.with_suffix(".so.tmp")
-    rb._run([hipcc, *rb.COMMON, *rb.HIP_FLAGS, "-shared", "-o", str(tmp), str(HERE / "pipeline_stages.hip")])
-    os.replace(tmp, LIB)
+    for src in ("pipeline_stages", "stack_stages"):
+        tmp = HERE / f"lib{src}.so.tmp"
+        rb._run([hipcc, *rb.COMMON, *rb.HIP_FLAGS, "-shared", "-o", str(tmp), str(HERE / f"{src}.hip")])
+        os.replace(tmp, HERE / f"lib{src}.so")
     return LIB
 
 
