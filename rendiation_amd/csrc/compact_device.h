@@ -61,8 +61,10 @@ __device__ __forceinline__ void block_compact2(bool ka, bool kb, uint32_t item, 
 }
 
 // Live blocks whose offsets k_scatter2 sums itself: at most 16 loads a thread,
-// where the scan launch takes 7 to 9 us (a preview frame of 4 bounces: 431 ->
-// 395 us); beyond that the sums, quadratic in the blocks, cost more.
+// where the scan launch takes 5 us and more (a preview frame of 3 bounces: 438
+// -> 411 us); beyond that the sums, quadratic in the blocks, cost more (a cull
+// pass of 512, 4096, 8192 and 16384 blocks: 21.2, 32.3, 44.5 and 72.6 us with
+// the scan, 16.1, 29.1, 46.9 and 93.1 without).
 constexpr uint32_t kDirectBlocks = 4096;
 
 constexpr uint32_t kScanThreads = 1024;

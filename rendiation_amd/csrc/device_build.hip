@@ -525,7 +525,9 @@ __global__ void k_median_sort(Dev d) {
 // serial chain of dependent scratch and global accesses: 12.6 ms for both trees
 // of 100k triangles; a wave per subtree takes 1.1 ms (a rebuild of the scene
 // 34.2 -> 21.2 ms).
-constexpr u32 kSmallNodes = 160;  // 2 kSmall - 1, and some for degenerate (empty) children
+// 2 kSmall - 1, and some for empty children (boxes whose areas overflow): trees with empty leaves are refused in any
+// case, here or when they are emitted
+constexpr u32 kSmallNodes = 160;
 
 __device__ __forceinline__ u32 rank_of(unsigned long long m) {
   return __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));

@@ -438,18 +438,21 @@ __device__ __forceinline__ uint32_t wave_count(bool v) {
 
 // Traces the slots [next, end) of the launch and every chunk that more(next,
 // end) gets after them (false: no more), refilling the wave when kRefill
-// lanes are idle.  Slots below n0 belong to the first segment.
+// lanes are idle (16 and 48 instead of 32: a 1080p frame 0.7 and 1.8 % slower,
+// a height-field step 0.5 and 3.0 %).  Slots below n0 belong to the first
+// segment.
 constexpr uint32_t kRefill = 32;
 // Inner steps go on while 1 / kKeep of the busy lanes want them.  Fewer lanes
 // waste vector instructions, more hold back the leaves whose hits shorten the
-// rays (2, 3, 4, 8: 366, 377, 431, 483 us for 1M rays in 100k triangles, but
-// 4.42, 4.15, 4.51, 4.50 ms for a batch of 16 scenes, measured on an earlier
-// build of these kernels).
+// rays (2, 4 and 8 instead of 3: 1M rays in 100k triangles 3.2, 1.6 and 9.3 %
+// slower, a batch of 16 scenes 0.8, 2.8 and 13.8 %, a 1080p frame 0.6, 0.5 and
+// 2.4 %).
 constexpr uint32_t kKeep = 3;
 // Leaves go before instances unless the lanes at instances outnumber those at
 // leaves by more than this: an instance step costs twice a leaf's, so it waits
-// for company (1, 2, 4: 500, 482, 474 us for a small-mesh material step, 15.96,
-// 15.86, 15.72 ms for a height-field step, 2.32, 2.26, 2.28 ms for a batch).
+// for company (1 and 5 instead of 3: a material step 0.9 and 0.3 % slower, a
+// batch of 16 scenes 2.8 and 1.1 %, a height-field step 1.2 % slower and 0.7 %
+// faster).
 constexpr uint32_t kLeavesFirst = 3;
 
 template <int K, int S, int B, bool CNT, int LAYOUT, class More>
@@ -669,9 +672,9 @@ __device__ __forceinline__ void trace_wave(const TraceParams &p, uint32_t n0, ui
 
 // The register bound of a launch that asks for occupancy (TraceTune::waves):
 // 96 registers, 5 waves per SIMD.  At 6 or 8 waves the kernels spill inside
-// their loops (1080p frame 1.86 ms at 5 waves, 1.95 at 6; ambient-occlusion
-// sample, whose launches are the cooperative kernel's, 468 us at 5, 487 at 4,
-// 535 at 6; 1M rays in 100k triangles 336 us at 5, 352 at 6, 427 at 4).
+// their loops (6 and 4 waves instead of 5: 1M rays in 100k triangles 3.4 and
+// 4.7 % slower, a 1080p frame 5.8 and 7.1 %, an ambient-occlusion sample, whose
+// launches are the cooperative kernel's, 10.5 and 4.9 %).
 constexpr int kWavesBound = 5;
 
 // Live slots of the first and the second segment of a launch.
@@ -713,8 +716,8 @@ constexpr uint32_t kCoopLanes = 8;
 constexpr uint32_t kCoopWideLanes = 16;
 constexpr uint32_t kCoopWideMax = 32768;
 // Inner steps go on while 1 / kCoopKeep of the wave's busy lanes want them
-// (2, 3, 6: 1.95, 1.97, 1.97 ms for the 1080p frame, 535, 538, 549 us for an
-// ambient-occlusion sample).
+// (3 and 6 instead of 2: a 1080p frame 0.3 and 1.4 % slower, an
+// ambient-occlusion sample 0.6 and 2.5 %).
 constexpr uint32_t kCoopKeep = 2;
 
 template <int G>
@@ -978,8 +981,9 @@ __global__ __launch_bounds__(B, W) void k_trace_persist(TraceParams p) {
   const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr uint32_t kWaves = B / 64u;
   const uint32_t share = (total / kWorkGroups + 63u) & ~63u;  // slots of one XCD, in whole chunks
-  // chunks of 64, larger when a wave has very many to pull, smaller when the
-  // first ones already leave waves without rays
+  // chunks of 64, larger when a wave has very many to pull (5M rays in 2000
+  // triangles: 390 us in chunks of 64, 358 of 128; 16M: 1170 and 1106), smaller
+  // when the first ones already leave waves without rays
   const uint32_t chunk = total >= (1u << 22) ? 128u : rays_per_wave(total, gridDim.x * kWaves);
   uint32_t tried = 0;      // shares found drained
   bool own = true;         // the first chunk is not taken yet
