@@ -507,7 +507,9 @@ typedef struct rdrt_tune {
                            refill lanes whose rays have ended */
   uint32_t cull;        /* 1 = a first pass finishes rays that miss their scene's root box and queues the rest */
   uint32_t wide;        /* node layout: 0 = child pairs (64 B), 1 = child quads (four boxes, 128 B),
-                           2 = quantized child quads (four 8-bit boxes, 64 B) */
+                           2 = quantized child quads (four 8-bit boxes, 64 B).  0 and 1 report a hit for the same
+                           rays; the wider boxes of 2 may add hits of rays that pass a box of triangles by less
+                           than their step */
   float ms;             /* rdrt_autotune: per-launch time of the chosen shape on the sample */
   uint32_t coop;        /* launches with at most this many live rays (device-side count) are traced by the
                            cooperative kernel, 8 lanes per ray (16 for launches of at most 32,768 live rays):
@@ -675,8 +677,10 @@ int32_t rdrt_pt_backward(rdrt_ctx *ctx, const float *adj_dev, float *grad_albedo
  * normal).  The paths are recomputed by replaying the frame, not stored.
  * grad_nrm_dev may be NULL when no geometry has vertex normals.  Same frame
  * conditions, adjoint layout and bit-reproducible sums as rdrt_pt_backward
- * (the replay keeps 48 bytes of gradient terms per path and bounce, and 12
- * bytes of sums per vertex component, in context scratch). */
+ * (the replay keeps 48 bytes of gradient terms per path and bounce, and 96
+ * bytes of sums per vertex, in context scratch).  The replay traces with the
+ * launch shape set when it runs: keep the node layout of the frame, another
+ * one may choose another of two hits at equal t. */
 int32_t rdrt_pt_backward_geometry(rdrt_ctx *ctx, const float *adj_dev, float *grad_positions_dev,
                                   float *grad_normals_dev);
 /* L2 loss helper: adj_dev[i] = 2 (a[i] - b[i]); *loss_dev (one f64) =

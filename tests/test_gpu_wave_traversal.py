@@ -108,7 +108,7 @@ def test_axis_parallel_rays(device):
     rays[np.arange(n), 4 + axis] = np.where(rng.random(n) < 0.5, 1.0, -1.0)
     neg = rng.random((n, 3)) < 0.5  # zeros of both signs
     rays[:, 4:7] = np.where((rays[:, 4:7] == 0.0) & neg, np.float32(-0.0), rays[:, 4:7])
-    rays[: n // 3, 4] += np.float32(1e-20)  # and components whose reciprocal is beyond the bound
+    rays[: n // 3, 4] += np.float32(1e-20)  # and tiny components, whose reciprocals are huge
     rays[:, 3], rays[:, 7] = 1e-4, 100.0
     want = _check(s, rays, "axis-parallel")
     assert np.count_nonzero(want[:, 0] != MISS) > 100
